@@ -292,13 +292,15 @@ int mea_qkvg_proj(const mea_desc* d, const void* x, const void* wq, const void* 
 
 namespace {
 
-int attn_fwd_launch(const mea_desc* d, const void* q, const void* k, const void* v, void* o, float* lse, float sl2e,
+int attn_fwd_launch(const mea_desc* d, const void* q, const void* k, const void* v, void* o, void* sig, float* lse,
+                    float sl2e,
                     const float* qk_norm2, const Varlen* var, void* stream) {
   mea::AttnFwdParams p;
   p.q = static_cast<const bf16_bits*>(q);
   p.k = static_cast<const bf16_bits*>(k);
   p.v = static_cast<const bf16_bits*>(v);
   p.o = static_cast<bf16_bits*>(o);
+  p.sig = static_cast<bf16_bits*>(sig);
   p.lse = lse;
   p.B = (int)d->B;
   p.H = (int)d->H;
@@ -319,7 +321,7 @@ int attn_fwd_impl(const mea_desc* d, const void* q, const void* k, const void* v
   if (rc != MEA_OK) return rc;
   rc = check_ptrs({q, k, v, o});
   if (rc != MEA_OK) return rc;
-  return attn_fwd_launch(d, q, k, v, o, lse, sl2e, qk_norm2, nullptr, stream);
+  return attn_fwd_launch(d, q, k, v, o, nullptr, lse, sl2e, qk_norm2, nullptr, stream);
 }
 
 int gate_oproj_launch(const mea_desc* d, const void* o, const void* sig, const void* wo, void* y, void* stream) {
@@ -400,7 +402,6 @@ int fwd_impl(const mea_desc* d, const Varlen* var, const void* x, const void* wq
   void* k = at<void>(ws, L.k);
   void* v = at<void>(ws, L.v);
   void* sig = at<void>(ws, L.sig);
-  void* o = o_save != nullptr ? o_save : at<void>(ws, L.o);
   // q is stored in log2 units; the projection records the largest q and k
   // row norms so the attention can take its fixed-offset softmax.
   float* qkn = at<float>(ws, L.qkn);
@@ -420,9 +421,11 @@ int fwd_impl(const mea_desc* d, const Varlen* var, const void* x, const void* wq
   rc = proj_launch(d, x, wq, wk, wv, wg, f1, f2, q, k, v, sig, nullptr, nullptr, nullptr, qs, qkn, tpos, tabp,
                    tab_rows, wpk, stream);
   if (rc != MEA_OK) return rc;
-  rc = attn_fwd_launch(d, q, k, v, o, lse_save, 1.0f, qkn, var, stream);
+  // O itself is written only where the backward needs it; z = O * sigmoid(a_g)
+  // takes the place of sigmoid(a_g).
+  rc = attn_fwd_launch(d, q, k, v, o_save, sig, lse_save, 1.0f, qkn, var, stream);
   if (rc != MEA_OK) return rc;
-  return gate_oproj_launch(d, o, sig, wo, y, stream);
+  return gate_oproj_launch(d, sig, nullptr, wo, y, stream);
 }
 
 // Buffers of one backward pass inside the workspace (and dx).

@@ -331,6 +331,21 @@ __global__ __launch_bounds__(256, N <= 64 ? 4 : N == 128 ? 3 : 1) void attn_fwd_
     main_loop(std::false_type{});
   }
 
+  // The output gate's rows are requested before the staging that they wait
+  // behind. Gating here rather than in the output projection's operand fetch
+  // reads one activation there instead of two and leaves its loop without the
+  // products: output projection 0.239 -> 0.202 ms, this kernel 0.988 -> 1.011 ms
+  // at B64 T4096 H8 N64; with few workgroups the projection gains most.
+  const size_t HN = (size_t)p.H * N;
+  constexpr int NOUT = QW * CH / 64;
+  u32x4 sgw[NOUT];
+  if (p.sig != nullptr) {
+#pragma unroll
+    for (int it = 0; it < NOUT; ++it) {
+      const int id = lane + 64 * it, t = min(q0w + id / CH, T - 1);
+      sgw[it] = ld16(p.sig + (tok_row0 + t) * HN + (size_t)hd * N + (id % CH) * 8);
+    }
+  }
   // Normalise, write lse and stage O^T (lane = query) as rows for 16-byte stores.
   bf16_bits* stg = smem + wave * QW * OP;
 #pragma unroll
@@ -349,14 +364,15 @@ __global__ __launch_bounds__(256, N <= 64 ? 4 : N == 128 ? 3 : 1) void attn_fwd_
       }
   }
   __syncthreads();
-  const size_t HN = (size_t)p.H * N;
 #pragma unroll
-  for (int it = 0; it < QW * CH / 64; ++it) {
+  for (int it = 0; it < NOUT; ++it) {
     const int id = lane + 64 * it, row = id / CH, dc = id % CH;
     const int t = q0w + row;
     if (t < T) {
       const u32x4 val = *reinterpret_cast<const u32x4*>(stg + row * OP + dc * 8);
-      st16(p.o + (tok_row0 + t) * HN + (size_t)hd * N + dc * 8, val);
+      const size_t off = (tok_row0 + t) * HN + (size_t)hd * N + dc * 8;
+      if (p.o != nullptr) st16(p.o + off, val);
+      if (p.sig != nullptr) st16(p.sig + off, gate8(val, sgw[it]));
     }
   }
 }

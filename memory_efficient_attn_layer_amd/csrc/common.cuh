@@ -131,6 +131,15 @@ __device__ __forceinline__ u32x4 pack8(const float* f) {
   return v;
 }
 
+// Elementwise product of 8 bf16 values (the output gate O * sigmoid(a_g)),
+// rounded to bf16.
+__device__ __forceinline__ u32x4 gate8(const u32x4& a, const u32x4& b) {
+  u32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = pack2(lo_bf(a[i]) * lo_bf(b[i]), hi_bf(a[i]) * hi_bf(b[i]));
+  return r;
+}
+
 __device__ __forceinline__ bf16x8 as_frag(const u32x4& v) { return __builtin_bit_cast(bf16x8, v); }
 // Concatenation of two 64-bit halves into one MFMA operand; written as a
 // shuffle so the two halves can be loaded straight into adjacent registers.

@@ -20,12 +20,13 @@ namespace mea {
 
 // ---------------------------------------------------------------------------
 // y = (O * sig) Wo^T, on the token-block main loop: A = Wo rows (output
-// features, k = HN), B = O * sig rows, gated while the slab is written to
-// LDS. A workgroup covers the NF output features from group * NF of BT
+// features, k = HN), B = O * sig rows: read as z = O * sig, which the attention
+// forward leaves, or (GATED, the stand-alone stage entry point) gated while
+// the slab is written to LDS. A workgroup covers the NF output features from group * NF of BT
 // tokens (the last group may reach past C); y rows leave through an LDS
 // staging block as whole-row segments.
 // ---------------------------------------------------------------------------
-template <int NF>
+template <int NF, bool GATED>
 __global__ __launch_bounds__(TokShape<NF>::NT, 1) void gate_oproj_kernel(OprojParams p) {
   using S = TokShape<NF>;
   constexpr int SP = 128 + 8;  // staging pitch (elements)
@@ -37,7 +38,7 @@ __global__ __launch_bounds__(TokShape<NF>::NT, 1) void gate_oproj_kernel(OprojPa
   const int ngrp = (C + NF - 1) / NF, lid = xcd_remap(blockIdx.x, gridDim.x);
   const int m0 = (lid / ngrp) * S::BT, f0 = (lid % ngrp) * NF;
   f32x4 acc[8][4];
-  tok_mainloop<NF, true>(HN, smem, p.wo + (size_t)f0 * HN, HN, 32, min(NF, C - f0), p.o, p.sig, HN, m0, M, acc);
+  tok_mainloop<NF, GATED>(HN, smem, p.wo + (size_t)f0 * HN, HN, 32, min(NF, C - f0), p.o, p.sig, HN, m0, M, acc);
 
   const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, g = lane >> 4;
   const int wave = tid >> 6, wf = wave % S::WF, wt = wave / S::WF;
@@ -63,7 +64,10 @@ __global__ __launch_bounds__(TokShape<NF>::NT, 1) void gate_oproj_kernel(OprojPa
 template <int NF>
 static void launch_oproj_nf(const OprojParams& p, hipStream_t s) {
   const dim3 grid(((p.M + TokShape<NF>::BT - 1) / TokShape<NF>::BT) * ((p.C + NF - 1) / NF));
-  hipLaunchKernelGGL(gate_oproj_kernel<NF>, grid, dim3(TokShape<NF>::NT), 0, s, p);
+  if (p.sig != nullptr)
+    hipLaunchKernelGGL((gate_oproj_kernel<NF, true>), grid, dim3(TokShape<NF>::NT), 0, s, p);
+  else
+    hipLaunchKernelGGL((gate_oproj_kernel<NF, false>), grid, dim3(TokShape<NF>::NT), 0, s, p);
 }
 
 hipError_t launch_gate_oproj(const OprojParams& p, hipStream_t s) {

@@ -51,7 +51,10 @@ hipError_t launch_token_positions(const int* cu, int nseq, int M, int* tpos, hip
 // Causal flash attention forward.
 struct AttnFwdParams {
   const bf16_bits *q, *k, *v;               // (B, H, T, N)
-  bf16_bits* o;                             // (B, T, H*N)
+  bf16_bits* o;                             // (B, T, H*N), or null (with sig)
+  // (B, T, H*N) sigmoid(a_g) in, z = O * sigmoid(a_g) out (the output
+  // projection's operand), or null.
+  bf16_bits* sig;
   float* lse;                               // (B, H, T) natural log, or null
   // Squared-norm bounds of the q and k rows (see ProjParams) or null. When
   // given and sl2e * |q| |k| <= kFixedBound, the softmax runs without a max.
@@ -109,7 +112,7 @@ struct TableGradParams {
 };
 hipError_t launch_table_grad(const TableGradParams& p, int N, hipStream_t s);
 
-// y = (o * sig) Wo^T.
+// y = (o * sig) Wo^T, or y = o Wo^T with sig null (o already gated).
 struct OprojParams {
   const bf16_bits *o, *sig;                 // (M, HN)
   const bf16_bits* wo;                      // (C, HN)

@@ -38,13 +38,6 @@ struct TokShape {
   static constexpr int SMEM = 2 * STAGE;
 };
 
-__device__ __forceinline__ u32x4 gate8(const u32x4& a, const u32x4& b) {
-  u32x4 r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) r[i] = pack2(lo_bf(a[i]) * lo_bf(b[i]), hi_bf(a[i]) * hi_bf(b[i]));
-  return r;
-}
-
 // Accumulates this wave's 128 x 64 block of D over the whole K into acc
 // (zeroed here). Rows of A past na - 1 read row na - 1 and rows of B past
 // M - 1 read row M - 1 (their results are not to be stored). K % 32 == 0.
