@@ -24,6 +24,7 @@ struct Layout {
   size_t wpk;                                // k-slab-major copies of Wq, Wk, Wv, Wg
   size_t dO, daq, dag;                       // backward (da_k, da_v overwrite k, v)
   size_t rx, rq, rk, delta, woT, wcatT, part;
+  size_t dxa, dxd;                           // tiled dx: fp32 rows, row dots (over part)
   size_t dak, dotq, dotk;                    // table gradients (MEA_PASS_BWD_TABLES): da_k beside k, row dots
   size_t total;
 };
@@ -60,6 +61,14 @@ Layout make_layout(const mea_desc& d, int pass) {
     L.woT = take(HN * C * 2);
     L.wcatT = take(C * 4 * HN * 2);
     L.part = take((size_t)mea::dw_splits((int)M, (int)C, (int)HN) * (4 * HN * C + C * HN) * 4);
+    if (mea::dx_tile_tokens((int)M, (int)C, (int)HN) != 0) {
+      // The tiled dx leaves fp32 rows and dot products for its second pass,
+      // over the dW partials (dead by then) and as far past them as needed.
+      const size_t rows = M * C * 4, dots = M * ((C + mea::kTileF - 1) / mea::kTileF) * 4;
+      L.dxa = L.part;
+      L.dxd = L.part + align_up(rows);
+      if (off < L.dxd + align_up(dots)) off = L.dxd + align_up(dots);
+    }
     if (pass == MEA_PASS_BWD_TABLES) {
       // The table gradients read k after the dK/dV kernel: da_k gets its own
       // rows, and the kernels leave one dot product per (b, h, t) row.
@@ -654,7 +663,9 @@ int bwd_impl(const mea_desc* d, const Varlen* var, const void* dy, const void* x
   // 768 < C <= 1024: feature groups of 512 over 128 tokens, group 0's
   // uncorrected rows parked in the recomputed q buffer (dead after the
   // attention backward; M x HN >= M x 512 elements).
-  dxp.scratch = C > 768 && C <= 1024 && HN >= 512 ? bf.q : nullptr;
+  dxp.scratch = mea::dx_two_groups(C, HN) ? bf.q : nullptr;
+  dxp.acc = at<float>(ws, L.dxa);
+  dxp.dotp = at<float>(ws, L.dxd);
   dxp.M = M;
   dxp.C = C;
   dxp.HN = HN;

@@ -13,6 +13,7 @@
 //   dW_p = (rx da_p)^T x   and   dx = acc - x * rx^2 * (acc . x) / C
 // with acc = sum_p (rx da_p) W_p; neither xh nor dxh is ever stored.
 #include "kernels.h"
+#include "rowops.cuh"
 #include "slab.cuh"
 #include "tokgemm.cuh"
 
@@ -62,12 +63,23 @@ __global__ __launch_bounds__(TokShape<NF>::NT, 1) void gate_oproj_kernel(OprojPa
 }
 
 template <int NF>
+static int tok_grid(int M, int F) {
+  return ((M + TokShape<NF>::BT - 1) / TokShape<NF>::BT) * ((F + NF - 1) / NF);
+}
+// The NF a feature count F runs with.
+static int tok_features(int F) { return F == 768 ? 768 : F % 512 == 0 ? 512 : 256; }
+static int tok_workgroups(int M, int F) {
+  const int nf = tok_features(F);
+  return nf == 768 ? tok_grid<768>(M, F) : nf == 512 ? tok_grid<512>(M, F) : tok_grid<256>(M, F);
+}
+
+template <int NF>
 static void launch_oproj_nf(const OprojParams& p, hipStream_t s) {
-  const dim3 grid(((p.M + TokShape<NF>::BT - 1) / TokShape<NF>::BT) * ((p.C + NF - 1) / NF));
+  const dim3 grid(tok_grid<NF>(p.M, p.C)), block(TokShape<NF>::NT);
   if (p.sig != nullptr)
-    hipLaunchKernelGGL((gate_oproj_kernel<NF, true>), grid, dim3(TokShape<NF>::NT), 0, s, p);
+    hipLaunchKernelGGL((gate_oproj_kernel<NF, true>), grid, block, 0, s, p);
   else
-    hipLaunchKernelGGL((gate_oproj_kernel<NF, false>), grid, dim3(TokShape<NF>::NT), 0, s, p);
+    hipLaunchKernelGGL((gate_oproj_kernel<NF, false>), grid, block, 0, s, p);
 }
 
 hipError_t launch_gate_oproj(const OprojParams& p, hipStream_t s) {
@@ -76,9 +88,12 @@ hipError_t launch_gate_oproj(const OprojParams& p, hipStream_t s) {
   // block to 64 and re-read all of Wo from L2 for every 64 tokens. A width
   // that is no multiple of 256 ends in a partial group (its Wo rows past
   // C - 1 read row C - 1, its stores stop at C).
-  if (p.C == 768)
+  if (const int tt = p.sig == nullptr ? tile_tokens(p.M, p.C, tok_workgroups(p.M, p.C)) : 0)
+    return launch_oproj_tile(p, tt, s);
+  const int nf = tok_features(p.C);
+  if (nf == 768)
     launch_oproj_nf<768>(p, s);
-  else if (p.C % 512 == 0)
+  else if (nf == 512)
     launch_oproj_nf<512>(p, s);
   else
     launch_oproj_nf<256>(p, s);
@@ -146,7 +161,7 @@ __global__ __launch_bounds__(TokShape<NF>::NT, 1) void dz_gate_bwd_kernel(DzPara
       const int j = f0 + wf * 128 + cc * 8;
       const bool valid = m < M && j < HN;
       const int mc = m < M ? m : M - 1, jc = j < HN ? j : 0;
-      float dz[8], sg[8], ov[8];
+      float dz[8];
       {
         const f32x4 a = *reinterpret_cast<const f32x4*>(stg + row * FP + cc * 8);
         const f32x4 c = *reinterpret_cast<const f32x4*>(stg + row * FP + cc * 8 + 4);
@@ -154,19 +169,9 @@ __global__ __launch_bounds__(TokShape<NF>::NT, 1) void dz_gate_bwd_kernel(DzPara
         for (int i = 0; i < 4; ++i) { dz[i] = a[i]; dz[4 + i] = c[i]; }
       }
       const size_t off = (size_t)mc * HN + jc;
-      unpack8(sgw[it], sg);
-      unpack8(ovw[it], ov);
-      const float rxv = rxw[it];
-      float dov[8], dag[8], zv[8], dl = 0.f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        // delta uses the bf16-rounded dO the attention backward consumes, so
-        // dP - delta cancels exactly where it should (a single key, T = 1).
-        dov[i] = bf2f(f2bf(dz[i] * sg[i]));
-        dag[i] = rxv * dz[i] * ov[i] * sg[i] * (1.0f - sg[i]);
-        zv[i] = ov[i] * sg[i];
-        dl += dov[i] * ov[i];
-      }
+      GateBwd r;
+      gate_bwd8(dz, sgw[it], ovw[it], rxw[it], r);
+      float dl = r.dl;
       dl += xor1(dl);
       dl += xor2(dl);
       if (N >= 64) dl += shfl_xor(dl, 4);  // N is uniform
@@ -184,9 +189,9 @@ __global__ __launch_bounds__(TokShape<NF>::NT, 1) void dz_gate_bwd_kernel(DzPara
         const int hh = jc / N, n = jc - hh * N;
         const int b = mc / T, t = mc - b * T;
         const size_t hrow = ((size_t)b * H + hh) * T + t;
-        st16(p.dO + hrow * N + n, pack8(dov));
-        st16(p.dag + (size_t)mc * p.ld_dag + jc, pack8(dag));
-        st16(p.sig + off, pack8(zv));  // sigmoid(a_g) is dead from here on
+        st16(p.dO + hrow * N + n, pack8(r.dov));
+        st16(p.dag + (size_t)mc * p.ld_dag + jc, pack8(r.dag));
+        st16(p.sig + off, pack8(r.zv));  // sigmoid(a_g) is dead from here on
         if (n == 0) p.delta[hrow] = dl;
       }
     }
@@ -195,28 +200,23 @@ __global__ __launch_bounds__(TokShape<NF>::NT, 1) void dz_gate_bwd_kernel(DzPara
 
 template <int NF>
 static void launch_dz_nf(const DzParams& p, int HN, hipStream_t s) {
-  const dim3 grid(((p.M + TokShape<NF>::BT - 1) / TokShape<NF>::BT) * ((HN + NF - 1) / NF));
-  hipLaunchKernelGGL(dz_gate_bwd_kernel<NF>, grid, dim3(TokShape<NF>::NT), 0, s, p);
+  hipLaunchKernelGGL(dz_gate_bwd_kernel<NF>, dim3(tok_grid<NF>(p.M, HN)), dim3(TokShape<NF>::NT), 0, s, p);
 }
 
 hipError_t launch_dz_gate_bwd(const DzParams& p, hipStream_t s) {
   const int HN = p.H * p.N;
   if (p.C % 32 != 0 || (p.N != 32 && p.N != 64 && p.N != 128 && p.N != 256)) return hipErrorInvalidValue;
   // Feature groups of 512 where HN allows (see launch_gate_oproj).
-  if (HN == 768)
+  // A 256-wide head does not fit a tile of the tiled form.
+  if (const int tt = p.N <= kTileF ? tile_tokens(p.M, HN, tok_workgroups(p.M, HN)) : 0) return launch_dz_tile(p, tt, s);
+  const int nf = tok_features(HN);
+  if (nf == 768)
     launch_dz_nf<768>(p, HN, s);
-  else if (HN % 512 == 0)
+  else if (nf == 512)
     launch_dz_nf<512>(p, HN, s);
   else
     launch_dz_nf<256>(p, HN, s);
   return hipGetLastError();
-}
-
-// Part `part` of da as a pointer, without branches or an indexed read (a
-// pointer picked by index from the parameters is read from a private copy).
-__device__ __forceinline__ const bf16_bits* da_part(const DaParts& dp, int part) {
-  auto m = [&](const bf16_bits* ptr, int i) { return (uint64_t)(uintptr_t)ptr & (0ull - (uint64_t)(part == i)); };
-  return reinterpret_cast<const bf16_bits*>((uintptr_t)(m(dp.q, 0) | m(dp.k, 1) | m(dp.v, 2) | m(dp.g, 3)));
 }
 
 // ---------------------------------------------------------------------------
@@ -420,9 +420,7 @@ __global__ __launch_bounds__(64 * ((CP / 128) * (8 % (CP / 128) == 0 ? 8 / (CP /
     float d = 0.f;
 #pragma unroll
     for (int fb = 0; fb < FB; ++fb) {
-      const u32x2 xw = *xs_at(tb * 16 + c16e, fb);
-      d += acc[fb][tb][0] * lo_bf(xw[0]) + acc[fb][tb][1] * hi_bf(xw[0]) + acc[fb][tb][2] * lo_bf(xw[1]) +
-           acc[fb][tb][3] * hi_bf(xw[1]);
+      d += dot4(acc[fb][tb], *xs_at(tb * 16 + c16e, fb));
     }
     d += shfl_xor(d, 16);
     d += shfl_xor(d, 32);
@@ -451,14 +449,14 @@ __global__ __launch_bounds__(64 * ((CP / 128) * (8 % (CP / 128) == 0 ? 8 / (CP /
 #pragma unroll
       for (int i = 0; i < WF; ++i) dot += dotp[i][wt * 64 + tb * 16 + c16e];
     }
-    const float cf = last ? rxr[tb] * rxr[tb] * dot * inv_c : 0.f;
+    const float cf = last ? dx_coef(rxr[tb], dot, inv_c) : 0.f;
 #pragma unroll
     for (int fb = 0; fb < FB; ++fb) {
       u32x2* xp = xs_at(tb * 16 + c16e, fb);
       const u32x2 xw = *xp;
       const f32x4& a = acc[fb][tb];
-      const float o0 = a[0] - lo_bf(xw[0]) * cf, o1 = a[1] - hi_bf(xw[0]) * cf;
-      const float o2 = a[2] - lo_bf(xw[1]) * cf, o3 = a[3] - hi_bf(xw[1]) * cf;
+      const float o0 = dx_apply(a[0], lo_bf(xw[0]), cf), o1 = dx_apply(a[1], hi_bf(xw[0]), cf);
+      const float o2 = dx_apply(a[2], lo_bf(xw[1]), cf), o3 = dx_apply(a[3], hi_bf(xw[1]), cf);
       *xp = u32x2{pack2(o0, o1), pack2(o2, o3)};
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's writes are done
@@ -491,12 +489,12 @@ __global__ __launch_bounds__(64 * ((CP / 128) * (8 % (CP / 128) == 0 ? 8 / (CP /
         if (m >= M) continue;
         const int col = wf * 128 + ch * 8;
         const float rxv = p.rx[m];
-        const float cf = rxv * rxv * dsum[wt * 64 + r] * inv_c;
+        const float cf = dx_coef(rxv, dsum[wt * 64 + r], inv_c);
         float a[8], xv[8], o[8];
         unpack8(ld16(p.scratch + (size_t)m * CP + col), a);
         unpack8(ld16(p.x + (size_t)m * C + col), xv);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = a[e] - xv[e] * cf;
+        for (int e = 0; e < 8; ++e) o[e] = dx_apply(a[e], xv[e], cf);
         st16(p.dx + (size_t)m * C + col, pack8(o));
       }
     }
@@ -627,8 +625,7 @@ __global__ __launch_bounds__(512, 1) void dx_wide_kernel(DxParams p) {
           const int f = f0 + wf * 128 + 16 * fb + 4 * g;
           if (f >= C) continue;
           const u32x2 xv = *reinterpret_cast<const u32x2*>(xg + (size_t)mrow[tb] * C + f);
-          d += acc[fb][tb][0] * lo_bf(xv[0]) + acc[fb][tb][1] * hi_bf(xv[0]) + acc[fb][tb][2] * lo_bf(xv[1]) +
-               acc[fb][tb][3] * hi_bf(xv[1]);
+          d += dot4(acc[fb][tb], xv);
         }
       }
       d += shfl_xor(d, 16);
@@ -651,15 +648,15 @@ __global__ __launch_bounds__(512, 1) void dx_wide_kernel(DxParams p) {
     for (int tb = 0; tb < TB; ++tb) {
       const int tl = tb * 16 + c16;
       const float rxv = p.rx[mrow[tb]];
-      const float cf = last ? rxv * rxv * dsum[tl] * inv_c : 0.f;
+      const float cf = last ? dx_coef(rxv, dsum[tl], inv_c) : 0.f;
 #pragma unroll
       for (int fb = 0; fb < FB; ++fb) {
         u32x2 xv = {0u, 0u};
         const int f = f0 + wf * 128 + 16 * fb + 4 * g;
         if (last && f < C) xv = *reinterpret_cast<const u32x2*>(xg + (size_t)mrow[tb] * C + f);
         const f32x4& a = acc[fb][tb];
-        const float o0 = a[0] - lo_bf(xv[0]) * cf, o1 = a[1] - hi_bf(xv[0]) * cf;
-        const float o2 = a[2] - lo_bf(xv[1]) * cf, o3 = a[3] - hi_bf(xv[1]) * cf;
+        const float o0 = dx_apply(a[0], lo_bf(xv[0]), cf), o1 = dx_apply(a[1], hi_bf(xv[0]), cf);
+        const float o2 = dx_apply(a[2], lo_bf(xv[1]), cf), o3 = dx_apply(a[3], hi_bf(xv[1]), cf);
         *reinterpret_cast<u32x2*>(stg + c16 * SP + 16 * fb + 4 * g) = u32x2{pack2(o0, o1), pack2(o2, o3)};
       }
       __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's staging writes are done
@@ -687,22 +684,28 @@ __global__ __launch_bounds__(512, 1) void dx_wide_kernel(DxParams p) {
         if (m >= M || f0 + wf * 128 >= C) continue;
         const size_t off = (size_t)m * C + f0 + wf * 128 + ch * 8;
         const float rxv = p.rx[m];
-        const float cf = rxv * rxv * dsum[tb * 16 + row] * inv_c;
+        const float cf = dx_coef(rxv, dsum[tb * 16 + row], inv_c);
         float a[8], xv[8], o[8];
         unpack8(ld16(p.dx + off), a);
         unpack8(ld16(xg + off), xv);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = a[e] - xv[e] * cf;
+        for (int e = 0; e < 8; ++e) o[e] = dx_apply(a[e], xv[e], cf);
         st16(p.dx + off, pack8(o));
       }
     }
   }
 }
 
+int dx_tile_tokens(int M, int C, int HN) {
+  const int bt = C <= 256 ? 256 : C <= 512 || dx_two_groups(C, HN) ? 128 : 64;  // tokens per workgroup in launch_dx
+  return tile_tokens(M, C, (M + bt - 1) / bt, C > 1024 ? 256 : 128);
+}
+
 hipError_t launch_dx(const DxParams& p, hipStream_t s) {
   // Model widths are multiples of 32; a width runs on the smallest padded
   // layout that holds it, widths past 1024 on the feature-group kernel.
   if (p.C < 32 || p.C % 32 != 0) return hipErrorInvalidValue;
+  if (const int tt = dx_tile_tokens(p.M, p.C, p.HN)) return launch_dx_tile(p, tt, s);
   if (p.C <= 256)
     hipLaunchKernelGGL(dx_kernel<256>, dim3((p.M + 255) / 256), dim3(512), 0, s, p);
   else if (p.C <= 512)

@@ -121,6 +121,16 @@ struct OprojParams {
 };
 hipError_t launch_gate_oproj(const OprojParams& p, hipStream_t s);
 
+// Tiled forms of the output projection, dZ and dx (tilegemm.hip): 128-feature
+// x tt-token tiles, for token counts that leave the row-owning kernels' grids
+// short of the chip.
+constexpr int kTileF = 128;
+// Tokens per tile (32, 64 or 128) for M tokens and F output features, or 0:
+// the row-owning kernel, whose grid has row_wgs workgroups, more than limit,
+// runs.
+int tile_tokens(int M, int F, int row_wgs, int limit = 128);
+hipError_t launch_oproj_tile(const OprojParams& p, int tt, hipStream_t s);
+
 // dZ = dy Wo, then the gate backward:
 //   dO = dZ * sig            -> (B, H, T, N)
 //   da_g = rx * dZ * O * sig * (1 - sig)   -> (M, HN), row stride ld_dag
@@ -139,6 +149,7 @@ struct DzParams {
   int M, T, C, H, N, ld_dag;
 };
 hipError_t launch_dz_gate_bwd(const DzParams& p, hipStream_t s);
+hipError_t launch_dz_tile(const DzParams& p, int tt, hipStream_t s);
 
 // The gradient of the four projection outputs, da = [da_q | da_k | da_v |
 // da_g] (M, 4*HN), rows pre-scaled by rx, as the dx and dW GEMMs read it:
@@ -161,8 +172,21 @@ struct DxParams {
   // 1024-wide layout over 64 tokens runs instead.
   bf16_bits* scratch;
   int M, C, HN;
+  // Tiled form (dx_tile_tokens > 0), else unused: acc (M, C) fp32 and the row
+  // dot products of every feature tile (M, ceil(C / kTileF)) fp32.
+  float *acc, *dotp;
 };
 hipError_t launch_dx(const DxParams& p, hipStream_t s);
+// Tokens per tile of the tiled form for this shape, or 0 (row-owning kernel).
+int dx_tile_tokens(int M, int C, int HN);
+hipError_t launch_dx_tile(const DxParams& p, int tt, hipStream_t s);
+// Whether the 512-wide layout walks 768 < C <= 1024 in two feature groups.
+__host__ __device__ constexpr bool dx_two_groups(int C, int HN) { return C > 768 && C <= 1024 && HN >= 512; }
+// Leading features whose accumulators the row-owning kernels park in bf16
+// before the RMSNorm correction (every feature group but the last).
+__host__ __device__ constexpr int dx_parked_features(int C, int HN) {
+  return C > 1024 ? (C - 1) / 1024 * 1024 : dx_two_groups(C, HN) ? 512 : 0;
+}
 
 // Weight gradients, split over tokens into fp32 partial sums:
 //   dWcat = da^T x        (4*HN, C)   da = [da_q | da_k | da_v | da_g]
