@@ -241,6 +241,27 @@ __host__ __device__ __forceinline__ int xcd_remap(int L, int G) {
   return start + i;
 }
 
+// Order of the output tiles of a GEMM of nt token tiles x nf feature tiles:
+// bands of `band` token tiles, feature by feature inside a band. The
+// workgroups an XCD runs at one time take consecutive tiles. With weights that
+// fit its 4 MB L2 they keep to whole token tiles (band 1: the activations come
+// from beyond L2 once, the weights stay). Larger weights would then be re-read
+// from beyond L2 for every few token tiles, so the tiles in flight cover a
+// near-square block instead (band 8: 8 x 8 of the projection's 64 per XCD).
+// Projection, band 1 / 8, us: C 2048 H 16 N 128 T 2048 92 / 72, T 16384 663 /
+// 509; C 1024 (8 MB) B4 T8192 324 / 310; C 512 (2 MB) B64 T2048 355 / 363.
+// Bands of 4, 16 and 32 lie within 4% of 8.
+struct TileIndex {
+  int t, f;
+};
+__host__ __device__ __forceinline__ int tile_band(int64_t weight_bytes) { return weight_bytes > (4 << 20) ? 8 : 1; }
+__host__ __device__ __forceinline__ TileIndex band_tile(int L, int nt, int nf, int band) {
+  const int b = L / (band * nf), r = L - b * (band * nf);
+  const int n = nt - b * band < band ? nt - b * band : band;  // token tiles of this band
+  const int f = r / n;
+  return TileIndex{b * band + (r - f * n), f};
+}
+
 // Work-item order of the attention kernels. Logical item l = head * nb + k,
 // where block k = 0 of a head is its heaviest (the most key or query tiles)
 // and k = nb - 1 its lightest. Each XCD runs a contiguous range of items

@@ -39,8 +39,7 @@
 
 namespace mea {
 
-// Tile coordinates of logical tile L (head-minor order, so the tiles of one
-// token tile are consecutive and share their x rows in L2).
+// Tile coordinates of logical tile L of ntt token tiles (see band_tile).
 struct ProjTile {
   int m0, h, f0;
 };
@@ -53,14 +52,14 @@ constexpr int kProjStages = 3;
 // N = 32: a tile holds the four projections of a head pair, h is the pair
 // (heads 2h and 2h + 1; H is even).
 template <int N>
-__device__ __forceinline__ ProjTile proj_tile(int L, int H) {
+__device__ __forceinline__ ProjTile proj_tile(int L, int ntt, int H, int band) {
   if constexpr (N == 32) {
-    const int np = H / 2, tt = L / np;
-    return ProjTile{tt * kProjBT, L - tt * np, 0};
+    const TileIndex ti = band_tile(L, ntt, H / 2, band);
+    return ProjTile{ti.t * kProjBT, ti.f, 0};
   } else {
     constexpr int NFT = 4 * N / kProjBF;
-    const int tt = L / (H * NFT), rem = L - tt * (H * NFT);
-    return ProjTile{tt * kProjBT, rem / NFT, (rem % NFT) * kProjBF};
+    const TileIndex ti = band_tile(L, ntt, H * NFT, band);
+    return ProjTile{ti.t * kProjBT, ti.f / NFT, (ti.f % NFT) * kProjBF};
   }
 }
 // Tiles of one 128-token tile: 4 * H * N stacked-weight rows in tiles of 256.
@@ -106,7 +105,8 @@ __global__ __launch_bounds__(256, 2) void qkvg_proj_kernel(ProjParams p) {
   const int wf = wave % WF, wt = wave / WF;
 
   // This workgroup's tiles: start + j0 + i * nj for i < ntl.
-  const int ntiles = ((M + BT - 1) / BT) * proj_tiles_per_token_tile(H, N);
+  const int band = tile_band((int64_t)8 * HN * C);
+  const int ntt = (M + BT - 1) / BT, ntiles = ntt * proj_tiles_per_token_tile(H, N);
   const int G = gridDim.x, xcd = blockIdx.x & 7, j0 = blockIdx.x >> 3;
   const int nj = (G - xcd + 7) >> 3;
   const int q8 = ntiles >> 3, r8 = ntiles & 7;
@@ -135,7 +135,7 @@ __global__ __launch_bounds__(256, 2) void qkvg_proj_kernel(ProjParams p) {
   // they do not evict the x slabs and weights from L2.
   int iss_ti = 0, iss_ks = 0, iss_st = 0, iss_rot = 0;
   auto plan_tile = [&](int ti) {
-    const ProjTile tl = proj_tile<N>(start + j0 + ti * nj, H);
+    const ProjTile tl = proj_tile<N>(start + j0 + ti * nj, ntt, H, band);
     iss_rot = tl.h % nk;
     if constexpr (N == 32) {
       // [q; v; k; g] of the head pair: rows 64h .. 64h + 63 of each matrix,
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(256, 2) void qkvg_proj_kernel(ProjParams p) {
   // published once after the last tile.
   float nmax = 0.f, nmax_k = 0.f;
   for (int ti = 0; ti < ntl; ++ti) {
-    const ProjTile tl = proj_tile<N>(start + j0 + ti * nj, H);
+    const ProjTile tl = proj_tile<N>(start + j0 + ti * nj, ntt, H, band);
 #pragma unroll
     for (int fb = 0; fb < FB; ++fb)
 #pragma unroll

@@ -25,15 +25,21 @@ namespace mea {
 
 namespace {
 
-// Tile of 128 features x TT tokens, four waves. A stage holds 64 k elements:
+// Waves per tile: two per SIMD for 128 tokens (dZ at M = 2048, C = H*N = 2048
+// 31.5 -> 28.9 us against one, output projection 25.6 -> 24.1, dx 82.8 -> 81.0);
+// for 64 tokens the wave tiles would shrink to 32 x 32 and dx runs 51 -> 54 us.
+template <int TT>
+constexpr int kTileWaves = TT == 128 ? 8 : 4;
+
+// Tile of 128 features x TT tokens. A stage holds 64 k elements:
 // two 32-wide weight sub-slabs (128 rows, 1 KB contiguous per load
 // instruction) and one 64-wide activation slab (TT rows of 128 bytes: whole
 // cache lines), laid out as slab.cuh describes.
 template <int TT>
 struct TileShape {
   static_assert(TT == 32 || TT == 64 || TT == 128, "tokens per tile");
-  static constexpr int FT = kTileF, NW = 4;
-  static constexpr int WT = TT == 32 ? 1 : 2, WF = NW / WT;   // waves along tokens, features
+  static constexpr int FT = kTileF, NW = kTileWaves<TT>, NT = 64 * NW;  // waves, threads
+  static constexpr int WT = TT == 32 ? 1 : TT * NW / 256, WF = NW / WT;  // waves along tokens, features
   static constexpr int FB = FT / WF / 16, TB = TT / WT / 16;  // 16-blocks per wave
   static constexpr int NA = FT / 16 / NW;                     // A load instructions per wave and sub-slab
   static constexpr int NB = TT / 8 / NW;                      // B load instructions per wave and stage
@@ -51,7 +57,7 @@ constexpr int vmcnt_imm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 // slab of k-steps 2 it and 2 it + 1; calls put(base, v) with a uniform base
 // and the lane offsets of this wave's load instructions (see tile_rows).
 //
-// One wave runs per SIMD, so the overlap is within the wave: the fragments of
+// One or two waves run per SIMD, so the overlap is within the wave: the fragments of
 // a sub-slab are read from LDS while the previous sub-slab's are multiplied,
 // across the stage boundary too (a stage is waited for half a stage before
 // its first product).
@@ -184,18 +190,15 @@ __device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
   }
 }
 
-// Tile (token block, feature tile) of workgroup blockIdx.x. The larger
-// operand is the one whose tiles an XCD keeps to itself: token-major (the
-// feature tiles of a token block run together on an XCD, every XCD reads the
-// weights) or feature-major (every XCD reads the activations).
+// Tile of workgroup blockIdx.x for F features of K (band_tile over each XCD's run of tiles).
 struct TilePos {
   int m0, f0;
 };
 template <int TT>
-__device__ __forceinline__ TilePos tile_pos(int M, int F, bool token_major) {
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int nf = (F + kTileF - 1) / kTileF, nt = (M + TT - 1) / TT;
-  return token_major ? TilePos{(lid / nf) * TT, (lid % nf) * kTileF} : TilePos{(lid % nt) * TT, (lid / nt) * kTileF};
+__device__ __forceinline__ TilePos tile_pos(int M, int F, int K) {
+  const TileIndex ti = band_tile(xcd_remap(blockIdx.x, gridDim.x), (M + TT - 1) / TT, (F + kTileF - 1) / kTileF,
+                                 tile_band((int64_t)2 * F * K));
+  return TilePos{ti.t * TT, ti.f * kTileF};
 }
 
 // Lane offsets (bytes) of this wave's B load instructions: tile row r of
@@ -206,18 +209,18 @@ __device__ __forceinline__ void tile_rows(uint32_t (&v)[TileShape<TT>::NB], int 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int j = 0; j < TileShape<TT>::NB; ++j) {
-    const int row = (j * 4 + wave) * 8 + (lane >> 3);
+    const int row = (j * TileShape<TT>::NW + wave) * 8 + (lane >> 3);
     v[j] = (uint32_t)row_off(min(m0 + row, M - 1), (lane & 7) ^ slab_swz<64>(row)) * 2u;
   }
 }
 
 // y = z Wo^T, one 128-feature x TT-token tile per workgroup.
 template <int TT>
-__global__ __launch_bounds__(256, 1) void oproj_tile_kernel(OprojParams p) {
+__global__ __launch_bounds__(TileShape<TT>::NT, 1) void oproj_tile_kernel(OprojParams p) {
   using S = TileShape<TT>;
   __shared__ __attribute__((aligned(16))) unsigned char smem[S::SMEM];
   const int M = p.M, C = p.C, HN = p.HN;
-  const TilePos tp = tile_pos<TT>(M, C, M >= C);
+  const TilePos tp = tile_pos<TT>(M, C, HN);
   const int m0 = tp.m0, f0 = tp.f0;
   uint32_t vb[S::NB];
   tile_rows<TT>(vb, m0, M, [&](int m, int c) { return (m - m0) * HN + 8 * c; });
@@ -229,8 +232,8 @@ __global__ __launch_bounds__(256, 1) void oproj_tile_kernel(OprojParams p) {
   const float* stg = tile_stage<TT>(smem, acc);
   const int tid = threadIdx.x, ch = tid & 15;
 #pragma unroll
-  for (int it = 0; it < TT / 16; ++it) {
-    const int row = it * 16 + (tid >> 4), m = m0 + row, f = f0 + ch * 8;
+  for (int it = 0; it < TT * 16 / S::NT; ++it) {
+    const int row = it * (S::NT / 16) + (tid >> 4), m = m0 + row, f = f0 + ch * 8;
     if (m >= M || f >= C) continue;
     float v[8];
     load8(stg + row * S::SP + ch * 8, v);
@@ -241,11 +244,11 @@ __global__ __launch_bounds__(256, 1) void oproj_tile_kernel(OprojParams p) {
 // dZ = dy Wo with the gate backward, as dz_gate_bwd_kernel, one tile per
 // workgroup (N <= 128: a tile's 128 features are whole heads).
 template <int TT>
-__global__ __launch_bounds__(256, 1) void dz_tile_kernel(DzParams p) {
+__global__ __launch_bounds__(TileShape<TT>::NT, 1) void dz_tile_kernel(DzParams p) {
   using S = TileShape<TT>;
   __shared__ __attribute__((aligned(16))) unsigned char smem[S::SMEM];
   const int M = p.M, C = p.C, H = p.H, T = p.T, N = p.N, HN = H * N;
-  const TilePos tp = tile_pos<TT>(M, HN, M >= HN);
+  const TilePos tp = tile_pos<TT>(M, HN, C);
   const int m0 = tp.m0, f0 = tp.f0;
   // A width that is an odd multiple of 32 ends in half a slab: its chunks 4
   // to 7 re-read chunks 0 to 3 (not multiplied).
@@ -265,12 +268,12 @@ __global__ __launch_bounds__(256, 1) void dz_tile_kernel(DzParams p) {
       acc);
   const int tid = threadIdx.x, ch = tid & 15, f = f0 + ch * 8;
   // The rows the gate backward reads are requested before the tile is staged.
-  constexpr int NP = TT / 16;
+  constexpr int RP = S::NT / 16, NP = TT / RP;  // rows per pass, passes
   u32x4 sgw[NP], ovw[NP];
   float rxw[NP];
 #pragma unroll
   for (int it = 0; it < NP; ++it) {
-    const int mc = min(m0 + it * 16 + (tid >> 4), M - 1);
+    const int mc = min(m0 + it * RP + (tid >> 4), M - 1);
     const size_t off = (size_t)mc * HN + (f < HN ? f : 0);
     sgw[it] = ld16(p.sig + off);
     ovw[it] = ld16(p.o + off);
@@ -279,7 +282,7 @@ __global__ __launch_bounds__(256, 1) void dz_tile_kernel(DzParams p) {
   const float* stg = tile_stage<TT>(smem, acc);
 #pragma unroll
   for (int it = 0; it < NP; ++it) {
-    const int row = it * 16 + (tid >> 4), m = m0 + row;
+    const int row = it * RP + (tid >> 4), m = m0 + row;
     float dz[8];
     load8(stg + row * S::SP + ch * 8, dz);
     GateBwd r;
@@ -305,13 +308,13 @@ __global__ __launch_bounds__(256, 1) void dz_tile_kernel(DzParams p) {
 // products acc . x in p.dotp; dx_finish_kernel applies the input RMSNorm
 // backward, which needs the dot product of the whole row.
 template <int TT>
-__global__ __launch_bounds__(256, 1) void dx_tile_kernel(DxParams p) {
+__global__ __launch_bounds__(TileShape<TT>::NT, 1) void dx_tile_kernel(DxParams p) {
   using S = TileShape<TT>;
   __shared__ __attribute__((aligned(16))) unsigned char smem[S::SMEM];
   const int M = p.M, C = p.C, HN = p.HN;
   const DaParts& dp = p.da;
   const int N = dp.N, T = dp.T;
-  const TilePos tp = tile_pos<TT>(M, C, M >= C);
+  const TilePos tp = tile_pos<TT>(M, C, 4 * HN);
   const int m0 = tp.m0, f0 = tp.f0;
   // Token rows: token-major da_g at stride ld_g, head-major parts at row
   // hm(m) (in units of N, from head 0 of batch 0); both relative to token m0.
@@ -360,8 +363,8 @@ __global__ __launch_bounds__(256, 1) void dx_tile_kernel(DxParams p) {
   // of the accumulator layout (16 fb + 4 g .. + 3).
   const int nft = (C + kTileF - 1) / kTileF;
 #pragma unroll
-  for (int it = 0; it < (TT + 63) / 64; ++it) {
-    const int row = it * 64 + (tid >> 2), g = tid & 3, m = m0 + row;
+  for (int it = 0; it < (TT * 4 + S::NT - 1) / S::NT; ++it) {
+    const int row = it * (S::NT / 4) + (tid >> 2), g = tid & 3, m = m0 + row;
     if (row >= TT || m >= M) continue;
     const bf16_bits* xr = p.x + (size_t)m * C + f0 + 4 * g;
     u32x2 xw[8];
@@ -378,8 +381,8 @@ __global__ __launch_bounds__(256, 1) void dx_tile_kernel(DxParams p) {
     if (g == 0) p.dotp[(size_t)m * nft + f0 / kTileF] = d;
   }
 #pragma unroll
-  for (int it = 0; it < TT / 8; ++it) {
-    const int row = it * 8 + (tid >> 5), f = f0 + 4 * (tid & 31), m = m0 + row;
+  for (int it = 0; it < TT * 32 / S::NT; ++it) {
+    const int row = it * (S::NT / 32) + (tid >> 5), f = f0 + 4 * (tid & 31), m = m0 + row;
     if (m >= M || f >= C) continue;
     *reinterpret_cast<f32x4*>(p.acc + (size_t)m * C + f) =
         *reinterpret_cast<const f32x4*>(stg + row * S::SP + 4 * (tid & 31));
@@ -435,33 +438,33 @@ int tile_tokens(int M, int F, int row_wgs, int limit) {
 hipError_t launch_oproj_tile(const OprojParams& p, int tt, hipStream_t s) {
   const dim3 grid(tile_grid(p.M, p.C, tt));
   if (tt == 128)
-    hipLaunchKernelGGL(oproj_tile_kernel<128>, grid, dim3(256), 0, s, p);
+    hipLaunchKernelGGL(oproj_tile_kernel<128>, grid, dim3(TileShape<128>::NT), 0, s, p);
   else if (tt == 64)
-    hipLaunchKernelGGL(oproj_tile_kernel<64>, grid, dim3(256), 0, s, p);
+    hipLaunchKernelGGL(oproj_tile_kernel<64>, grid, dim3(TileShape<64>::NT), 0, s, p);
   else
-    hipLaunchKernelGGL(oproj_tile_kernel<32>, grid, dim3(256), 0, s, p);
+    hipLaunchKernelGGL(oproj_tile_kernel<32>, grid, dim3(TileShape<32>::NT), 0, s, p);
   return hipGetLastError();
 }
 
 hipError_t launch_dz_tile(const DzParams& p, int tt, hipStream_t s) {
   const dim3 grid(tile_grid(p.M, p.H * p.N, tt));
   if (tt == 128)
-    hipLaunchKernelGGL(dz_tile_kernel<128>, grid, dim3(256), 0, s, p);
+    hipLaunchKernelGGL(dz_tile_kernel<128>, grid, dim3(TileShape<128>::NT), 0, s, p);
   else if (tt == 64)
-    hipLaunchKernelGGL(dz_tile_kernel<64>, grid, dim3(256), 0, s, p);
+    hipLaunchKernelGGL(dz_tile_kernel<64>, grid, dim3(TileShape<64>::NT), 0, s, p);
   else
-    hipLaunchKernelGGL(dz_tile_kernel<32>, grid, dim3(256), 0, s, p);
+    hipLaunchKernelGGL(dz_tile_kernel<32>, grid, dim3(TileShape<32>::NT), 0, s, p);
   return hipGetLastError();
 }
 
 hipError_t launch_dx_tile(const DxParams& p, int tt, hipStream_t s) {
   const dim3 grid(tile_grid(p.M, p.C, tt));
   if (tt == 128)
-    hipLaunchKernelGGL(dx_tile_kernel<128>, grid, dim3(256), 0, s, p);
+    hipLaunchKernelGGL(dx_tile_kernel<128>, grid, dim3(TileShape<128>::NT), 0, s, p);
   else if (tt == 64)
-    hipLaunchKernelGGL(dx_tile_kernel<64>, grid, dim3(256), 0, s, p);
+    hipLaunchKernelGGL(dx_tile_kernel<64>, grid, dim3(TileShape<64>::NT), 0, s, p);
   else
-    hipLaunchKernelGGL(dx_tile_kernel<32>, grid, dim3(256), 0, s, p);
+    hipLaunchKernelGGL(dx_tile_kernel<32>, grid, dim3(TileShape<32>::NT), 0, s, p);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int64_t n = (int64_t)p.M * (p.C / 8);
