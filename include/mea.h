@@ -202,6 +202,14 @@ int mea_bwd_varlen(const mea_desc* d, const int32_t* cu_seqlens, int32_t nseq,
                    size_t ws_bytes, void* stream);
 
 /*
+ * fp32 copies of rows 0..rows-1 of two bf16 rotary tables (rows x N, N a
+ * multiple of 8, contiguous), in one launch: the tables cross this interface
+ * as fp32 arrays.
+ */
+int mea_table_rows(const void* f1, const void* f2, int64_t rows, int64_t N,
+                   float* f1_out, float* f2_out, void* stream);
+
+/*
  * Prefill of a KV cache: the inference forward of a whole prompt (mea_fwd
  * with o_save = lse_save = NULL, same workspace) that also copies the
  * prompt's k and v rows, exactly as the attention consumed them, into rows

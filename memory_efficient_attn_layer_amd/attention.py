@@ -126,6 +126,18 @@ def _pad_heads(H: int, N: int, weights, factor1, factor2, pad_n: int, pad_h: int
 
 
 def _tables32(factor1: torch.Tensor, factor2: torch.Tensor, T: int):
+    """fp32 copies of the first T rows of both tables (one launch for
+    contiguous bf16 tables, the reference's own dtype)."""
+    if (factor1.dtype == factor2.dtype == torch.bfloat16 and factor1.is_contiguous() and factor2.is_contiguous()
+            and (factor1.data_ptr() | factor2.data_ptr()) % 16 == 0):
+        N, dev = factor1.shape[1], factor1.device
+        out = torch.empty((2, T, N), device=dev, dtype=torch.float32)
+        f1, f2 = out[0], out[1]
+        with torch.cuda.device(dev):
+            rc = _lib.load().mea_table_rows(factor1.data_ptr(), factor2.data_ptr(), T, N, f1.data_ptr(), f2.data_ptr(),
+                                            _lib.stream_of(dev))
+        _lib.check(rc, "mea_table_rows")
+        return f1, f2
     return factor1[:T].float().contiguous(), factor2[:T].float().contiguous()
 
 

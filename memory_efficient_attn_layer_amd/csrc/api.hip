@@ -166,14 +166,14 @@ T* at(void* ws, size_t off) {
 
 // ---- kernel timing diagnostics -------------------------------------------
 enum KernelId {
-  K_QKVG_PROJ, K_ATTN_FWD, K_GATE_OPROJ, K_TRANSPOSE, K_ZERO, K_DZ_GATE_BWD,
+  K_QKVG_PROJ, K_ATTN_FWD, K_GATE_OPROJ, K_PREP, K_DZ_GATE_BWD,
   K_ATTN_BWD_DQ, K_ATTN_BWD_DKDV, K_DW_PARTIAL, K_DW_REDUCE, K_DX,
-  K_ATTN_DECODE, K_DECODE_COMBINE, K_SKINNY_GEMM, K_DECODE_PROJ, K_TABLE_GRAD, K_ROTARY_PACK, K_WEIGHT_PACK, K_COUNT
+  K_ATTN_DECODE, K_DECODE_COMBINE, K_SKINNY_GEMM, K_DECODE_PROJ, K_TABLE_GRAD, K_COUNT
 };
 const char* const kKernelNames[K_COUNT] = {
-    "qkvg_proj", "attn_fwd", "gate_oproj", "transpose", "zero_f32", "dz_gate_bwd",
+    "qkvg_proj", "attn_fwd", "gate_oproj", "prep", "dz_gate_bwd",
     "attn_bwd_dq", "attn_bwd_dkdv", "dw_partial", "dw_reduce", "dx",
-    "attn_decode", "attn_decode_combine", "skinny_gemm", "decode_proj", "table_grad", "rotary_pack", "weight_pack"};
+    "attn_decode", "attn_decode_combine", "skinny_gemm", "decode_proj", "table_grad"};
 
 struct ProfRec {
   int kernel;
@@ -235,8 +235,8 @@ float q_log2_scale(int64_t N) { return (float)(1.4426950408889634 / sqrt((double
 int64_t n_active(const mea_desc* d) { return d->N_active != 0 ? d->N_active : d->N; }
 
 // Launch sequence pieces; the public entry points validate before calling.
-// Packed tables (tabp, tab_rows rows; see pack_tables) or null: f1 / f2.
-// wpk: the k-slab-major weight copies (see pack_weights) or null: the
+// Packed tables (tabp, tab_rows rows; see prepare) or null: f1 / f2.
+// wpk: the k-slab-major weight copies (see prepare) or null: the
 // row-major weights wq .. wg.
 int proj_launch(const mea_desc* d, const void* x, const void* wq, const void* wk, const void* wv, const void* wg,
                 const float* f1, const float* f2, void* q, void* k, void* v, void* sig, float* rx, float* rq,
@@ -368,32 +368,43 @@ int mea_gate_oproj(const mea_desc* d, const void* o, const void* sig, const void
 
 namespace {
 
-// With d->tables_bf16: packs the table rows the projection reads (0 .. T-1;
-// packed sequences 0 .. max_len-1) into the workspace and returns the copy in
-// *tabp and its row count in *rows; otherwise *tabp = null.
-hipError_t pack_tables(const mea_desc* d, const Varlen* var, const float* f1, const float* f2, void* ws,
-                       const Layout& L, hipStream_t s, const bf16_bits** tabp, int* rows) {
-  *tabp = nullptr;
-  *rows = 0;
-  if (d->tables_bf16 == 0) return hipSuccess;
-  bf16_bits* out = at<bf16_bits>(ws, L.rot);
-  const int n = var != nullptr ? var->max_len : (int)d->T;
-  const hipError_t e = timed(K_ROTARY_PACK, s, [&] { return mea::launch_rotary_pack(f1, f2, n, (int)d->N, out, s); });
-  *tabp = out;
-  *rows = n;
-  return e;
-}
-
-// Wq, Wk, Wv, Wg into k-slab-major copies in the workspace (2 * 4HN * C
-// bytes) for the projection's weight-slab loads; returns the copy.
-hipError_t pack_weights(const mea_desc* d, const void* wq, const void* wk, const void* wv, const void* wg, void* ws,
-                        const Layout& L, hipStream_t s, const bf16_bits** wpk) {
-  bf16_bits* out = at<bf16_bits>(ws, L.wpk);
-  mea::WcatPackParams wp{static_cast<const bf16_bits*>(wq), static_cast<const bf16_bits*>(wk),
-                         static_cast<const bf16_bits*>(wv), static_cast<const bf16_bits*>(wg), out,
-                         (int)(d->H * d->N), (int)d->C};
-  *wpk = out;
-  return timed(K_WEIGHT_PACK, s, [&] { return mea::launch_wslab_pack(wp, s); });
+// What the projection and (backward) the GEMMs behind it read besides the
+// caller's arrays: the launch of launch_prep for a pass, and the pointers it
+// leaves. Table rows: 0 .. T-1, packed sequences 0 .. max_len-1.
+struct Prep {
+  const bf16_bits *tabp = nullptr, *wpk = nullptr;
+  int tab_rows = 0;
+  const int* tpos = nullptr;
+};
+hipError_t prepare(const mea_desc* d, const Varlen* var, const void* wq, const void* wk, const void* wv,
+                   const void* wg, const void* wo, const float* f1, const float* f2, void* ws, const Layout& L,
+                   float* zero2, bf16_bits* wcatT, bf16_bits* woT, hipStream_t s, Prep* out) {
+  mea::PrepParams p = {};
+  p.wq = static_cast<const bf16_bits*>(wq);
+  p.wk = static_cast<const bf16_bits*>(wk);
+  p.wv = static_cast<const bf16_bits*>(wv);
+  p.wg = static_cast<const bf16_bits*>(wg);
+  p.wo = static_cast<const bf16_bits*>(wo);
+  p.HN = (int)(d->H * d->N);
+  p.C = (int)d->C;
+  p.M = (int)(d->B * d->T);
+  if (mea::proj_wants_slabs(p.M, (int)d->H, (int)d->N)) out->wpk = p.wslab = at<bf16_bits>(ws, L.wpk);
+  p.wcatT = wcatT;
+  p.woT = woT;
+  if (d->tables_bf16 != 0) {
+    out->tab_rows = var != nullptr ? var->max_len : (int)d->T;
+    p.f1 = f1;
+    p.f2 = f2;
+    p.table_words = out->tab_rows * (int)(d->N / 4);
+    out->tabp = p.tabp = at<bf16_bits>(ws, L.rot);
+  }
+  p.zero2 = zero2;
+  if (var != nullptr) {
+    p.cu = var->cu;
+    p.nseq = var->nseq;
+    out->tpos = p.tpos = at<int>(ws, L.tpos);
+  }
+  return timed(K_PREP, s, [&] { return mea::launch_prep(p, s); });
 }
 
 int fwd_impl(const mea_desc* d, const Varlen* var, const void* x, const void* wq, const void* wk, const void* wv,
@@ -414,21 +425,12 @@ int fwd_impl(const mea_desc* d, const Varlen* var, const void* x, const void* wq
   // q is stored in log2 units; the projection records the largest q and k
   // row norms so the attention can take its fixed-offset softmax.
   float* qkn = at<float>(ws, L.qkn);
-  MEA_TRY(timed(K_ZERO, static_cast<hipStream_t>(stream),
-                [&] { return mea::launch_zero_f32(qkn, 2, static_cast<hipStream_t>(stream)); }));
   const float qs = q_log2_scale(n_active(d));
-  int* tpos = nullptr;
-  if (var != nullptr) {
-    tpos = at<int>(ws, L.tpos);
-    MEA_TRY(mea::launch_token_positions(var->cu, var->nseq, (int)d->T, tpos, static_cast<hipStream_t>(stream)));
-  }
-  const bf16_bits* tabp;
-  int tab_rows;
-  MEA_TRY(pack_tables(d, var, f1, f2, ws, L, static_cast<hipStream_t>(stream), &tabp, &tab_rows));
-  const bf16_bits* wpk;
-  MEA_TRY(pack_weights(d, wq, wk, wv, wg, ws, L, static_cast<hipStream_t>(stream), &wpk));
-  rc = proj_launch(d, x, wq, wk, wv, wg, f1, f2, q, k, v, sig, nullptr, nullptr, nullptr, qs, qkn, tpos, tabp,
-                   tab_rows, wpk, stream);
+  Prep pr;
+  MEA_TRY(prepare(d, var, wq, wk, wv, wg, wo, f1, f2, ws, L, qkn, nullptr, nullptr, static_cast<hipStream_t>(stream),
+                  &pr));
+  rc = proj_launch(d, x, wq, wk, wv, wg, f1, f2, q, k, v, sig, nullptr, nullptr, nullptr, qs, qkn, pr.tpos, pr.tabp,
+                   pr.tab_rows, pr.wpk, stream);
   if (rc != MEA_OK) return rc;
   // O itself is written only where the backward needs it; z = O * sigmoid(a_g)
   // takes the place of sigmoid(a_g).
@@ -482,30 +484,16 @@ int bwd_front(const mea_desc* d, const Varlen* var, const void* dy, const void* 
               const float* lse_save, float* df1, float* df2, const BwdBufs& bf, void* ws, void* stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int M = (int)(d->B * d->T), T = (int)d->T, H = (int)d->H, N = (int)d->N, C = (int)d->C;
-  const int HN = H * N;
   const Layout L = make_layout(*d, df1 != nullptr ? MEA_PASS_BWD_TABLES : MEA_PASS_BWD);
 
-  // Weight transposes (k-contiguous B operands for dZ and dx).
-  MEA_TRY(timed(K_TRANSPOSE, s, [&] { return mea::launch_transpose_slabs(static_cast<const bf16_bits*>(wo), C, HN, HN, bf.woT, s); }));
-  {
-    mea::WcatPackParams wp{static_cast<const bf16_bits*>(wq), static_cast<const bf16_bits*>(wk),
-                           static_cast<const bf16_bits*>(wv), static_cast<const bf16_bits*>(wg), bf.wcatT, HN, C};
-    MEA_TRY(timed(K_TRANSPOSE, s, [&] { return mea::launch_wcat_pack(wp, s); }));
-  }
+  // Weight transposes (k-contiguous operands for dZ and dx) and the layouts of
+  // the recompute.
+  Prep pr;
+  MEA_TRY(prepare(d, var, wq, wk, wv, wg, wo, f1, f2, ws, L, nullptr, bf.wcatT, bf.woT, s, &pr));
   // Recompute q, k, v, sigmoid(g) and the three RMS statistics.
   const float qs = q_log2_scale(n_active(d));
-  int* tpos = nullptr;
-  if (var != nullptr) {
-    tpos = at<int>(ws, L.tpos);
-    MEA_TRY(mea::launch_token_positions(var->cu, var->nseq, T, tpos, s));
-  }
-  const bf16_bits* tabp;
-  int tab_rows;
-  MEA_TRY(pack_tables(d, var, f1, f2, ws, L, s, &tabp, &tab_rows));
-  const bf16_bits* wpk;
-  MEA_TRY(pack_weights(d, wq, wk, wv, wg, ws, L, s, &wpk));
-  int rc = proj_launch(d, x, wq, wk, wv, wg, f1, f2, bf.q, bf.k, bf.v, bf.sig, bf.rx, bf.rq, bf.rk, qs, nullptr, tpos,
-                       tabp, tab_rows, wpk, stream);
+  int rc = proj_launch(d, x, wq, wk, wv, wg, f1, f2, bf.q, bf.k, bf.v, bf.sig, bf.rx, bf.rq, bf.rk, qs, nullptr,
+                       pr.tpos, pr.tabp, pr.tab_rows, pr.wpk, stream);
   if (rc != MEA_OK) return rc;
 
   mea::DzParams dz;
@@ -730,6 +718,16 @@ int mea_bwd_stage_grads(const mea_desc* d, const void* dy, const void* x, const 
   MEA_TRY(hipMemcpyAsync(dav, bf.v, act, hipMemcpyDeviceToDevice, s));
   MEA_TRY(hipMemcpyAsync(dO, bf.dO, act, hipMemcpyDeviceToDevice, s));
   MEA_TRY(hipMemcpyAsync(delta, bf.delta, stat, hipMemcpyDeviceToDevice, s));
+  return MEA_OK;
+}
+
+int mea_table_rows(const void* f1, const void* f2, int64_t rows, int64_t N, float* f1_out, float* f2_out,
+                   void* stream) {
+  const int rc = check_ptrs({f1, f2, f1_out, f2_out});
+  if (rc != MEA_OK) return rc;
+  if (rows < 1 || N < 8 || N % 8 != 0 || rows > (INT64_C(1) << 31) / N - 1) return MEA_ERR_SHAPE;
+  MEA_TRY(mea::launch_table_rows(static_cast<const bf16_bits*>(f1), static_cast<const bf16_bits*>(f2), (int)(rows * N),
+                                 f1_out, f2_out, static_cast<hipStream_t>(stream)));
   return MEA_OK;
 }
 

@@ -223,7 +223,7 @@ hipError_t launch_dz_gate_bwd(const DzParams& p, hipStream_t s) {
 // dx = rmsnorm_bwd([da_q|da_k|da_v|da_g] Wcat), one workgroup owns full rows.
 //
 // Computed transposed, D^T = Wcat^T da^T: A = Wcat^T rows (C features, k =
-// 4HN, stored k-slab-major by wcat_pack_kernel so that a slab is one
+// 4HN, stored k-slab-major by the prep kernel so that a slab is one
 // contiguous block), B = da rows (tokens). A 32-wide k-slab of da lies in one
 // head of one part (N >= 64): each slab has one base address, and a lane's
 // row offset from it, the same in every slab, is precomputed for the
@@ -1020,126 +1020,6 @@ hipError_t launch_dw_reduce(const DwReduceParams& p, hipStream_t s) {
   const size_t total = (size_t)4 * p.HN * p.C + (size_t)p.C * p.HN;
   const int G = (int)((total / 4 + 255) / 256);
   hipLaunchKernelGGL(dw_reduce_kernel, dim3(G), dim3(256), 0, s, p);
-  return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// Small helpers.
-// ---------------------------------------------------------------------------
-// SLABS: out is k-slab-major instead, element (c, r) of the transpose at
-// (r / 32) * cols * 32 + c * 32 + r % 32 (ld_out and col_off unused).
-template <bool SLABS>
-__global__ __launch_bounds__(256) void transpose_kernel(const bf16_bits* in, int rows, int cols, int ld_in,
-                                                        bf16_bits* out, int ld_out, int col_off) {
-  __shared__ bf16_bits tile[64][65];
-  const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  for (int r = ty; r < 64; r += 4) {
-    const int rr = r0 + r, cc = c0 + tx;
-    tile[r][tx] = (rr < rows && cc < cols) ? in[(size_t)rr * ld_in + cc] : (bf16_bits)0;
-  }
-  __syncthreads();
-  for (int c = ty; c < 64; c += 4) {
-    const int cc = c0 + c, rr = r0 + tx;
-    if (cc < cols && rr < rows) {
-      if (SLABS)
-        out[(size_t)(rr >> 5) * cols * 32 + (size_t)cc * 32 + (rr & 31)] = tile[tx][c];
-      else
-        out[(size_t)cc * ld_out + col_off + rr] = tile[tx][c];
-    }
-  }
-}
-
-hipError_t launch_transpose(const bf16_bits* in, int rows, int cols, int ld_in, bf16_bits* out, int ld_out,
-                            int col_off, hipStream_t s) {
-  hipLaunchKernelGGL(transpose_kernel<false>, dim3((cols + 63) / 64, (rows + 63) / 64), dim3(256), 0, s, in, rows,
-                     cols, ld_in, out, ld_out, col_off);
-  return hipGetLastError();
-}
-
-hipError_t launch_transpose_slabs(const bf16_bits* in, int rows, int cols, int ld_in, bf16_bits* out, hipStream_t s) {
-  if (rows % 32 != 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(transpose_kernel<true>, dim3((cols + 63) / 64, (rows + 63) / 64), dim3(256), 0, s, in, rows,
-                     cols, ld_in, out, 0, 0);
-  return hipGetLastError();
-}
-
-// Wcat^T in k-slab-major order (the dx A operand): element (f, k) at
-// (k / 32) * C * 32 + f * 32 + k % 32, k indexing the stacked rows of
-// [Wq; Wk; Wv; Wg] (part blockIdx.z, rows z * HN ..). A 64 x 64 tile of one
-// part goes through LDS; each thread writes 16-byte chunks (8 consecutive k
-// of one feature), so every 32-k slab of the tile leaves as 64 contiguous
-// 64-byte rows.
-__global__ __launch_bounds__(256) void wcat_pack_kernel(WcatPackParams p) {
-  __shared__ bf16_bits tile[64][64 + 2];  // [k][f]
-  const int z = blockIdx.z, HN = p.HN, C = p.C;
-  const bf16_bits* in = z == 0 ? p.wq : z == 1 ? p.wk : z == 2 ? p.wv : p.wg;  // (HN, C)
-  const int k0 = blockIdx.y * 64, f0 = blockIdx.x * 64, tid = threadIdx.x;
-#pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    const int i = tid + 256 * it, r = i >> 3, c = (i & 7) * 8;
-    u32x4 v = {0u, 0u, 0u, 0u};
-    if (k0 + r < HN && f0 + c < C) v = ld16(in + (size_t)(k0 + r) * C + f0 + c);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      tile[r][c + 2 * e] = (bf16_bits)(v[e] & 0xFFFFu);
-      tile[r][c + 2 * e + 1] = (bf16_bits)(v[e] >> 16);
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    // i = (slab half s, feature f, chunk ch): consecutive threads write consecutive 16-byte chunks.
-    const int i = tid + 256 * it, s = i >> 8, f = (i >> 2) & 63, ch = i & 3;
-    const int kl = s * 32 + ch * 8;
-    if (k0 + kl >= HN || f0 + f >= C) continue;
-    u32x4 v;
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      v[e] = (uint32_t)tile[kl + 2 * e][f] | ((uint32_t)tile[kl + 2 * e + 1][f] << 16);
-    const int k = z * HN + k0 + kl;  // HN and k0 are multiples of 32
-    st16(p.out + (size_t)(k >> 5) * C * 32 + (size_t)(f0 + f) * 32 + (k & 31), v);
-  }
-}
-
-hipError_t launch_wcat_pack(const WcatPackParams& p, hipStream_t s) {
-  if (p.HN % 32 != 0 || p.C % 8 != 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(wcat_pack_kernel, dim3((p.C + 63) / 64, (p.HN + 63) / 64, 4), dim3(256), 0, s, p);
-  return hipGetLastError();
-}
-
-namespace {
-
-// One thread per 16-byte chunk of the packed output: matrix blockIdx.z,
-// k-slab kk, row r, chunk c8 (8 elements) <- row r, columns 32 kk + 8 c8.
-__global__ __launch_bounds__(256) void wslab_pack_kernel(WcatPackParams p) {
-  const int i = blockIdx.x * 256 + threadIdx.x;  // chunk index within one matrix
-  const int nch = p.HN * (p.C / 8);
-  if (i >= nch) return;
-  const int c8 = i & 3, r = (i >> 2) % p.HN, kk = (i >> 2) / p.HN;
-  const bf16_bits* w = blockIdx.z == 0 ? p.wq : blockIdx.z == 1 ? p.wk : blockIdx.z == 2 ? p.wv : p.wg;
-  const u32x4 v = ld16(w + (size_t)r * p.C + kk * 32 + c8 * 8);
-  *reinterpret_cast<u32x4*>(p.out + (size_t)blockIdx.z * p.HN * p.C + (size_t)i * 8) = v;
-}
-
-}  // namespace
-
-hipError_t launch_wslab_pack(const WcatPackParams& p, hipStream_t s) {
-  if (p.C % 32 != 0) return hipErrorInvalidValue;
-  const int nch = p.HN * (p.C / 8);
-  hipLaunchKernelGGL(wslab_pack_kernel, dim3((nch + 255) / 256, 1, 4), dim3(256), 0, s, p);
-  return hipGetLastError();
-}
-
-__global__ __launch_bounds__(256) void zero_f32_kernel(float* p, size_t n) {
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) p[i] = 0.f;
-}
-
-hipError_t launch_zero_f32(float* p, size_t n, hipStream_t s) {
-  if (n == 0) return hipSuccess;
-  size_t G = (n + 255) / 256;
-  if (G > 4096) G = 4096;
-  hipLaunchKernelGGL(zero_f32_kernel, dim3((unsigned)G), dim3(256), 0, s, p, n);
   return hipGetLastError();
 }
 

@@ -13,8 +13,8 @@ typedef uint16_t bf16_bits;
 struct ProjParams {
   const bf16_bits* x;                       // (M, C)
   // (H*N, C) weights: element (row, k) at row * w_row + (k / 32) * w_slab +
-  // k % 32. Row-major: w_row = C, w_slab = 32; the k-slab-major copy of
-  // launch_wslab_pack: w_row = 32, w_slab = 32 * H*N.
+  // k % 32. Row-major: w_row = C, w_slab = 32; the k-slab-major copies of
+  // launch_prep: w_row = 32, w_slab = 32 * H*N.
   const bf16_bits *wq, *wk, *wv, *wg;
   int w_row;
   int64_t w_slab;
@@ -41,12 +41,35 @@ struct ProjParams {
 };
 hipError_t launch_qkvg_proj(const ProjParams& p, int N, hipStream_t s);
 
-// tabp (ProjParams) from rows 0 .. rows-1 of f1 and f2: values rounded to
-// bf16, so exact for tables whose values are bf16 numbers.
-hipError_t launch_rotary_pack(const float* f1, const float* f2, int rows, int N, bf16_bits* tabp, hipStream_t s);
+// Whether the projection of M tokens wants k-slab-major weight copies.
+bool proj_wants_slabs(int M, int H, int N);
 
-// tpos[m] = m - cu[s] for cu[s] <= m < cu[s+1] (packed sequences).
-hipError_t launch_token_positions(const int* cu, int nseq, int M, int* tpos, hipStream_t s);
+// The layouts a pass builds before its first GEMM; null outputs are skipped.
+struct PrepParams {
+  const bf16_bits *wq, *wk, *wv, *wg;       // (HN, C)
+  const bf16_bits* wo;                      // (C, HN)
+  int HN, C;
+  // Wq, Wk, Wv, Wg each k-slab-major (C / 32, HN, 32), matrix i at i * HN * C:
+  // a 32-wide k-slab of any run of rows is one contiguous block.
+  bf16_bits* wslab;
+  // [Wq; Wk; Wv; Wg]^T for dx: element (f, k) at (k / 32) * C * 32 + f * 32 +
+  // k % 32, k over the stacked rows; and Wo^T for dZ likewise (C / 32, HN, 32).
+  bf16_bits *wcatT, *woT;
+  // tabp (ProjParams) from the first table_words 4-feature groups of f1 and
+  // f2: rounded to bf16, so exact for tables whose values are bf16 numbers.
+  const float *f1, *f2;
+  int table_words;
+  bf16_bits* tabp;
+  float* zero2;                             // two floats to clear
+  // tpos[m] = m - cu[s] for cu[s] <= m < cu[s+1] (packed sequences).
+  const int* cu;
+  int nseq, M;
+  int* tpos;
+};
+hipError_t launch_prep(const PrepParams& p, hipStream_t s);
+
+// The first n elements (a multiple of 8) of two bf16 tables as fp32.
+hipError_t launch_table_rows(const bf16_bits* f1, const bf16_bits* f2, int n, float* o1, float* o2, hipStream_t s);
 
 // Causal flash attention forward.
 struct AttnFwdParams {
@@ -210,34 +233,6 @@ struct DwReduceParams {
   int C, HN, splits;
 };
 hipError_t launch_dw_reduce(const DwReduceParams& p, hipStream_t s);
-
-// out(cols, rows) = in(rows, cols)^T for a bf16 matrix with leading
-// dimension ld_in; writes into out with leading dimension ld_out starting at
-// column col_off.
-hipError_t launch_transpose(const bf16_bits* in, int rows, int cols, int ld_in, bf16_bits* out,
-                            int ld_out, int col_off, hipStream_t s);
-// The same transpose stored k-slab-major: element (c, r) of out at
-// (r / 32) * cols * 32 + c * 32 + r % 32 (rows a multiple of 32).
-hipError_t launch_transpose_slabs(const bf16_bits* in, int rows, int cols, int ld_in, bf16_bits* out, hipStream_t s);
-
-// Wcat^T for dx in k-slab-major order: element (f, k) at
-// (k / 32) * C * 32 + f * 32 + k % 32, k over the stacked rows of
-// [Wq; Wk; Wv; Wg] (each (HN, C)).
-struct WcatPackParams {
-  const bf16_bits *wq, *wk, *wv, *wg;
-  bf16_bits* out;
-  int HN, C;
-};
-hipError_t launch_wcat_pack(const WcatPackParams& p, hipStream_t s);
-
-// Each of Wq, Wk, Wv, Wg (HN, C) into k-slab-major (C / 32, HN, 32) at
-// out + i * HN * C (i = 0 q, 1 k, 2 v, 3 g): a 32-wide k-slab of any run of
-// rows is one contiguous block, so the projection's weight-slab loads read
-// 1 KB of contiguous memory per instruction.
-hipError_t launch_wslab_pack(const WcatPackParams& p, hipStream_t s);
-
-// Fills n floats with zero (a kernel, so it is safe inside captured graphs).
-hipError_t launch_zero_f32(float* p, size_t n, hipStream_t s);
 
 // KV-cache decode step: one new token per sequence at position pos[b]
 // attends to cache rows 0 .. pos[b] (its own k / v included).

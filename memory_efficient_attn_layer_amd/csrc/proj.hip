@@ -16,11 +16,11 @@
 //
 // Tile: 256 features x 128 tokens. k-slabs of 32 stream through a 3-stage
 // LDS ring filled by direct global->LDS loads, two slabs ahead, continuously
-// across the tiles a workgroup walks (one barrier per slab). The block entry
-// points pass k-slab-major copies of the weights (a slab of a tile's rows is
-// one contiguous block, 1 KB per load instruction; from the row-major
-// matrices each instruction gathers 16 rows of 64 bytes): 0.714 -> 0.680 ms
-// per launch at B64 T4096 C512 H8 N64. Four waves of
+// across the tiles a workgroup walks (one barrier per slab). For more than one
+// round of tiles the block entry points pass k-slab-major copies of the weights
+// (a slab of a tile's rows is one contiguous block, 1 KB per load instruction;
+// from the row-major matrices each instruction gathers 16 rows of 64 bytes):
+// 0.714 -> 0.680 ms per launch at B64 T4096 C512 H8 N64. Four waves of
 // 128 features x 64 tokens (32 accumulators of 16x16): for N = 64 a wave owns
 // one rotary projection (q or k) and one plain one (v or g) of its tokens, so
 // the epilogue work is the same in every wave. Two workgroups share a CU, so
@@ -554,6 +554,15 @@ static void launch_proj_n(const ProjParams& p, int G, hipStream_t s) {
     hipLaunchKernelGGL((qkvg_proj_kernel<N, true, true>), dim3(G), dim3(256), 0, s, p);
 }
 
+// One round of workgroups (two per CU) reads each weight slab at most a few
+// times: a k-slab-major copy costs what its loads save. Pack + projection
+// against row-major, us: C 2048 H 16 N 128 T 700 11.8 + 51.6 / 52.5, T 2048 (512
+// tiles) 11.9 + 76.4 / 88.1; C 1024 H 16 N 64 B8 T512 (512 tiles) 4.8 + 52.8 /
+// 56.7; C 768 H 6 N 128 B3 T999 4.0 + 36.0 / 39.1, and a launch less.
+bool proj_wants_slabs(int M, int H, int N) {
+  return ((M + kProjBT - 1) / kProjBT) * proj_tiles_per_token_tile(H, N) > 512;
+}
+
 hipError_t launch_qkvg_proj(const ProjParams& p, int N, hipStream_t s) {
   if (N == 32 && p.H % 2 != 0) return hipErrorInvalidValue;  // tiles hold head pairs
   const int G = persistent_grid(((p.M + kProjBT - 1) / kProjBT) * proj_tiles_per_token_tile(p.H, N), 2);
@@ -567,52 +576,6 @@ hipError_t launch_qkvg_proj(const ProjParams& p, int N, hipStream_t s) {
     launch_proj_n<256>(p, G, s);
   else
     return hipErrorInvalidValue;
-  return hipGetLastError();
-}
-
-namespace {
-
-// One thread per 4-feature group i = t * N/4 + n/4 of rows 0 .. rows-1:
-// (f1[4i .. 4i+3], f2[4i .. 4i+3]) rounded to bf16 into word i.
-__global__ __launch_bounds__(256) void rotary_pack_kernel(const f32x4* f1, const f32x4* f2, int groups, u32x4* out) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= groups) return;
-  const f32x4 a = f1[i], b = f2[i];
-  out[i] = u32x4{pack2(a[0], a[1]), pack2(a[2], a[3]), pack2(b[0], b[1]), pack2(b[2], b[3])};
-}
-
-}  // namespace
-
-hipError_t launch_rotary_pack(const float* f1, const float* f2, int rows, int N, bf16_bits* tabp, hipStream_t s) {
-  const int groups = rows * (N / 4);
-  hipLaunchKernelGGL(rotary_pack_kernel, dim3((groups + 255) / 256), dim3(256), 0, s,
-                     reinterpret_cast<const f32x4*>(f1), reinterpret_cast<const f32x4*>(f2), groups,
-                     reinterpret_cast<u32x4*>(tabp));
-  return hipGetLastError();
-}
-
-namespace {
-
-// One thread per token: the sequence holding token m by binary search over
-// the nseq + 1 offsets cu (cu[0] = 0, increasing).
-__global__ __launch_bounds__(256) void token_positions_kernel(const int* cu, int nseq, int M, int* tpos) {
-  const int m = blockIdx.x * 256 + threadIdx.x;
-  if (m >= M) return;
-  int lo = 0, hi = nseq;  // cu[lo] <= m < cu[hi]
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (cu[mid] <= m)
-      lo = mid;
-    else
-      hi = mid;
-  }
-  tpos[m] = m - cu[lo];
-}
-
-}  // namespace
-
-hipError_t launch_token_positions(const int* cu, int nseq, int M, int* tpos, hipStream_t s) {
-  hipLaunchKernelGGL(token_positions_kernel, dim3((M + 255) / 256), dim3(256), 0, s, cu, nseq, M, tpos);
   return hipGetLastError();
 }
 

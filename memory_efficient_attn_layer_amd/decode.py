@@ -22,7 +22,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .attention import MAX_C_FORWARD, SUPPORTED_HEAD_DIMS, _pad_heads, _validate, storage_shape
+from .attention import MAX_C_FORWARD, SUPPORTED_HEAD_DIMS, _pad_heads, _tables32, _validate, storage_shape
 
 
 def cache_width(N: int, H: int) -> int:
@@ -82,7 +82,7 @@ def _padded(H: int, N: int, weights, factor1, factor2):
 def _tables(factor1, factor2, rows: int):
     if factor1.shape[0] < rows:
         raise ValueError(f"rotary tables have {factor1.shape[0]} rows, fewer than the cache capacity {rows}")
-    return factor1[:rows].float().contiguous(), factor2[:rows].float().contiguous()
+    return _tables32(factor1, factor2, rows)
 
 
 def prefill(x, q_weight, k_weight, v_weight, g_weight, o_weight, factor1, factor2, H: int, N: int,

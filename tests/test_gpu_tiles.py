@@ -3,6 +3,7 @@ their tiles, and against the row-owning forms that larger calls take."""
 import pytest
 import torch
 
+from memory_efficient_attn_layer_amd.attention import _tables32
 from memory_efficient_attn_layer_amd.synthetic import Workload, make_inputs
 from tests.parity_util import check_block, gpu_block
 
@@ -34,3 +35,25 @@ def test_tiled_and_row_owning_forms_return_the_same_bits(B, C, H, N):
         one = dict(inp, x=inp["x"][b:b + 1], dy=inp["dy"][b:b + 1])
         got = gpu_block(one, H, N, table_grad=False)
         assert torch.equal(got["y"], full["y"][b:b + 1]) and torch.equal(got["dx"], full["dx"][b:b + 1])
+
+
+def test_projection_from_packed_and_row_major_weights_is_the_same():
+    """512 projection tiles (64 x 128 tokens, 8 heads of 64) read the weights
+    row-major, 520 from k-slab-major copies."""
+    w = Workload(99, "tiles", 65, 128, 96, 8, 64)
+    inp = make_inputs(w, seed=7)
+    full = gpu_block(inp, 8, 64, table_grad=False)
+    part = gpu_block(dict(inp, x=inp["x"][:64], dy=inp["dy"][:64]), 8, 64, table_grad=False)
+    assert torch.equal(part["y"], full["y"][:64]) and torch.equal(part["dx"], full["dx"][:64])
+
+
+@pytest.mark.parametrize("T,N,rows", [(1, 32, 1), (77, 64, 77), (300, 16, 129), (513, 256, 512)])
+def test_table_rows_are_the_fp32_values(T, N, rows):
+    g = torch.Generator("cuda").manual_seed(T)
+    f1, f2 = (torch.randn(T, N, device="cuda", generator=g).bfloat16() for _ in range(2))
+    o1, o2 = _tables32(f1, f2, rows)
+    assert torch.equal(o1, f1[:rows].float()) and torch.equal(o2, f2[:rows].float())
+    # Tables the launch does not take (strided, unaligned) go through torch.
+    wide = torch.randn(T, 2 * N, device="cuda", generator=g).bfloat16()
+    o1, o2 = _tables32(wide[:, :N], wide[:, N:], rows)
+    assert torch.equal(o1, wide[:rows, :N].float()) and torch.equal(o2, wide[:rows, N:].float())
