@@ -96,8 +96,9 @@ __global__ __launch_bounds__(256, N <= 64 ? 4 : N == 128 ? 3 : 1) void attn_fwd_
   const int q0w = qi * BQ + wave * QW;
   const int kv_end = min(T, qi * BQ + BQ);
   const size_t head_off = head_row0 * N;
-  const bf16_bits* kg = p.k + head_off;
-  const bf16_bits* vg = p.v + head_off;
+  const size_t kv_off = VARLEN ? head_off : (size_t)bh * p.kv_T * N;
+  const bf16_bits* kg = p.k + kv_off;
+  const bf16_bits* vg = p.v + kv_off;
 
   bool fixed = false;
   if (p.qk_norm2 != nullptr && p.sl2e == 1.0f) {

@@ -254,7 +254,10 @@ __host__ __device__ __forceinline__ int xcd_remap(int L, int G) {
 struct TileIndex {
   int t, f;
 };
-__host__ __device__ __forceinline__ int tile_band(int64_t weight_bytes) { return weight_bytes > (4 << 20) ? 8 : 1; }
+constexpr int kTileBand = 8;
+__host__ __device__ __forceinline__ int tile_band(int64_t weight_bytes) {
+  return weight_bytes > (4 << 20) ? kTileBand : 1;
+}
 __host__ __device__ __forceinline__ TileIndex band_tile(int L, int nt, int nf, int band) {
   const int b = L / (band * nf), r = L - b * (band * nf);
   const int n = nt - b * band < band ? nt - b * band : band;  // token tiles of this band

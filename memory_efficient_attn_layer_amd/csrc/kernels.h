@@ -23,7 +23,8 @@ struct ProjParams {
   // n / 4 of row t = f1[t, n..n+3], f2[t, n..n+3]), or null: the epilogue
   // then reads f1 / f2. Used when every table value is a bf16 number.
   const bf16_bits* tabp;
-  bf16_bits *q, *k, *v;                     // (B, H, T, N)
+  bf16_bits *q, *k, *v;                     // (B, H, T, N); k and v: kv_T rows per head, the first T written
+  int kv_T;                                 // T, or the capacity of the KV cache they are
   bf16_bits* sig;                           // (M, H*N)
   float* rx;                                // (M) or null
   float *rq, *rk;                           // (B, H, T) or null
@@ -73,7 +74,8 @@ hipError_t launch_table_rows(const bf16_bits* f1, const bf16_bits* f2, int n, fl
 
 // Causal flash attention forward.
 struct AttnFwdParams {
-  const bf16_bits *q, *k, *v;               // (B, H, T, N)
+  const bf16_bits *q, *k, *v;               // (B, H, T, N); k and v: kv_T >= T rows per head
+  int kv_T;                                 // (not read for packed sequences)
   bf16_bits* o;                             // (B, T, H*N), or null (with sig)
   // (B, T, H*N) sigmoid(a_g) in, z = O * sigmoid(a_g) out (the output
   // projection's operand), or null.

@@ -53,14 +53,9 @@ constexpr int kProjStages = 3;
 // (heads 2h and 2h + 1; H is even).
 template <int N>
 __device__ __forceinline__ ProjTile proj_tile(int L, int ntt, int H, int band) {
-  if constexpr (N == 32) {
-    const TileIndex ti = band_tile(L, ntt, H / 2, band);
-    return ProjTile{ti.t * kProjBT, ti.f, 0};
-  } else {
-    constexpr int NFT = 4 * N / kProjBF;
-    const TileIndex ti = band_tile(L, ntt, H * NFT, band);
-    return ProjTile{ti.t * kProjBT, ti.f / NFT, (ti.f % NFT) * kProjBF};
-  }
+  constexpr int NFT = N == 32 ? 1 : 4 * N / kProjBF;
+  const TileIndex ti = band_tile(L, ntt, N == 32 ? H / 2 : H * NFT, band);
+  return ProjTile{ti.t * kProjBT, ti.f / NFT, (ti.f % NFT) * kProjBF};
 }
 // Tiles of one 128-token tile: 4 * H * N stacked-weight rows in tiles of 256.
 __host__ __device__ __forceinline__ int proj_tiles_per_token_tile(int H, int N) { return H * 4 * N / kProjBF; }
@@ -72,7 +67,10 @@ __host__ __device__ __forceinline__ int proj_tiles_per_token_tile(int H, int N) 
 // separate instantiation, so the (B, T) kernel keeps its code.
 // PK: the epilogue reads the packed bf16 tables p.tabp (one 16-byte load per
 // 4 features for both tables) instead of the fp32 f1 / f2 rows (two).
-template <int N, bool POS, bool PK>
+// EXT: tiles may run in bands of token tiles (see band_tile) and k, v may be a
+// KV cache (kv_T rows per head); an instantiation of its own, since both cost
+// the plain call 1% (58 spilled scalar registers instead of 37).
+template <int N, bool POS, bool PK, bool EXT>
 __global__ __launch_bounds__(256, 2) void qkvg_proj_kernel(ProjParams p) {
   constexpr int BT = kProjBT, BF = kProjBF, BK = kProjBK, NS = kProjStages;
   constexpr int STAGE = (BF + BT) * BK;
@@ -105,7 +103,7 @@ __global__ __launch_bounds__(256, 2) void qkvg_proj_kernel(ProjParams p) {
   const int wf = wave % WF, wt = wave / WF;
 
   // This workgroup's tiles: start + j0 + i * nj for i < ntl.
-  const int band = tile_band((int64_t)8 * HN * C);
+  const int band = EXT ? tile_band((int64_t)8 * HN * C) : 1;
   const int ntt = (M + BT - 1) / BT, ntiles = ntt * proj_tiles_per_token_tile(H, N);
   const int G = gridDim.x, xcd = blockIdx.x & 7, j0 = blockIdx.x >> 3;
   const int nj = (G - xcd + 7) >> 3;
@@ -455,10 +453,11 @@ __global__ __launch_bounds__(256, 2) void qkvg_proj_kernel(ProjParams p) {
     };
     auto drain_pj = [&](int gi, int tb) {
       const int pj = proj_of(gi), hg = head_of(gi);
+      const int rows = !EXT || pj == 0 ? T : p.kv_T;  // rows per head (q; k and v)
       if (pj < 2)
-        drain(gi, tb, (pj == 0 ? p.q : p.k) + (size_t)hg * T * N + col, (size_t)H * T * N, (size_t)N);
+        drain(gi, tb, (pj == 0 ? p.q : p.k) + (size_t)hg * rows * N + col, (size_t)H * rows * N, (size_t)N);
       else if (pj == 2)
-        drain(gi, tb, p.v + (size_t)hg * T * N + col, (size_t)H * T * N, (size_t)N);
+        drain(gi, tb, p.v + (size_t)hg * rows * N + col, (size_t)H * rows * N, (size_t)N);
       else
         drain(gi, tb, p.sig + (size_t)hg * N + col, (size_t)T * HN, (size_t)HN);
     };
@@ -541,17 +540,26 @@ int persistent_grid(int tiles, int per_cu) {
   return tiles < per_cu * cus[dev] ? tiles : per_cu * cus[dev];
 }
 
-template <int N>
+template <int N, bool EXT>
 static void launch_proj_n(const ProjParams& p, int G, hipStream_t s) {
   const bool pos = p.tpos != nullptr, pk = p.tabp != nullptr;
   if (!pos && !pk)
-    hipLaunchKernelGGL((qkvg_proj_kernel<N, false, false>), dim3(G), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((qkvg_proj_kernel<N, false, false, EXT>), dim3(G), dim3(256), 0, s, p);
   else if (!pos)
-    hipLaunchKernelGGL((qkvg_proj_kernel<N, false, true>), dim3(G), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((qkvg_proj_kernel<N, false, true, EXT>), dim3(G), dim3(256), 0, s, p);
   else if (!pk)
-    hipLaunchKernelGGL((qkvg_proj_kernel<N, true, false>), dim3(G), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((qkvg_proj_kernel<N, true, false, EXT>), dim3(G), dim3(256), 0, s, p);
   else
-    hipLaunchKernelGGL((qkvg_proj_kernel<N, true, true>), dim3(G), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((qkvg_proj_kernel<N, true, true, EXT>), dim3(G), dim3(256), 0, s, p);
+}
+
+template <int N>
+static void launch_proj(const ProjParams& p, hipStream_t s) {
+  const int G = persistent_grid(((p.M + kProjBT - 1) / kProjBT) * proj_tiles_per_token_tile(p.H, N), 2);
+  if (tile_band((int64_t)8 * p.H * N * p.C) > 1 || p.kv_T != p.T)
+    launch_proj_n<N, true>(p, G, s);
+  else
+    launch_proj_n<N, false>(p, G, s);
 }
 
 // One round of workgroups (two per CU) reads each weight slab at most a few
@@ -565,15 +573,14 @@ bool proj_wants_slabs(int M, int H, int N) {
 
 hipError_t launch_qkvg_proj(const ProjParams& p, int N, hipStream_t s) {
   if (N == 32 && p.H % 2 != 0) return hipErrorInvalidValue;  // tiles hold head pairs
-  const int G = persistent_grid(((p.M + kProjBT - 1) / kProjBT) * proj_tiles_per_token_tile(p.H, N), 2);
   if (N == 32)
-    launch_proj_n<32>(p, G, s);
+    launch_proj<32>(p, s);
   else if (N == 64)
-    launch_proj_n<64>(p, G, s);
+    launch_proj<64>(p, s);
   else if (N == 128)
-    launch_proj_n<128>(p, G, s);
+    launch_proj<128>(p, s);
   else if (N == 256)
-    launch_proj_n<256>(p, G, s);
+    launch_proj<256>(p, s);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();

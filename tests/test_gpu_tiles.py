@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from memory_efficient_attn_layer_amd.attention import _tables32
+from memory_efficient_attn_layer_amd.decode import KVCache, prefill
 from memory_efficient_attn_layer_amd.synthetic import Workload, make_inputs
 from tests.parity_util import check_block, gpu_block
 
@@ -57,3 +58,19 @@ def test_table_rows_are_the_fp32_values(T, N, rows):
     wide = torch.randn(T, 2 * N, device="cuda", generator=g).bfloat16()
     o1, o2 = _tables32(wide[:, :N], wide[:, N:], rows)
     assert torch.equal(o1, wide[:rows, :N].float()) and torch.equal(o2, wide[:rows, N:].float())
+
+
+@pytest.mark.parametrize("H,N", [(2, 32), (3, 64), (2, 128), (1, 256)], ids=lambda v: str(v))
+def test_prefill_writes_its_rows_of_the_cache_only(H, N):
+    B, T, C, cap = 2, 130, 96, 200
+    w = Workload(99, "prefill", B, cap, C, H, N)
+    inp = {k: v.cuda() for k, v in make_inputs(w, seed=N).items()}
+    x = inp["x"][:, :T].contiguous()
+    args = [inp[n] for n in ("wq", "wk", "wv", "wg", "wo", "f1", "f2")]
+    big, tight = (KVCache.empty(B, H, N, c, "cuda") for c in (cap, T))
+    for t in (big.k, big.v):
+        t.fill_(7.0)
+    yb, yt = prefill(x, *args, H, N, big), prefill(x, *args, H, N, tight)
+    assert torch.equal(yb, yt)
+    for a, b in ((big.k, tight.k), (big.v, tight.v)):
+        assert torch.equal(a[:, :, :T], b) and bool((a[:, :, T:] == 7.0).all())
