@@ -168,12 +168,12 @@ T* at(void* ws, size_t off) {
 enum KernelId {
   K_QKVG_PROJ, K_ATTN_FWD, K_GATE_OPROJ, K_PREP, K_DZ_GATE_BWD,
   K_ATTN_BWD_DQ, K_ATTN_BWD_DKDV, K_DW_PARTIAL, K_DW_REDUCE, K_DX,
-  K_ATTN_DECODE, K_DECODE_COMBINE, K_SKINNY_GEMM, K_DECODE_PROJ, K_TABLE_GRAD, K_COUNT
+  K_ATTN_DECODE, K_DECODE_COMBINE, K_SKINNY_GEMM, K_TABLE_GRAD, K_COUNT
 };
 const char* const kKernelNames[K_COUNT] = {
     "qkvg_proj", "attn_fwd", "gate_oproj", "prep", "dz_gate_bwd",
     "attn_bwd_dq", "attn_bwd_dkdv", "dw_partial", "dw_reduce", "dx",
-    "attn_decode", "attn_decode_combine", "skinny_gemm", "decode_proj", "table_grad"};
+    "attn_decode", "attn_decode_combine", "skinny_gemm", "table_grad"};
 
 struct ProfRec {
   int kernel;
@@ -760,24 +760,24 @@ int mea_prefill(const mea_desc* d, const void* x, const void* wq, const void* wk
 namespace {
 
 // Decode workspace: the raw products [a_q|a_k|a_v|a_g] (B x 4HN fp32), the
-// new token's q, sigmoid(g) and attention output (B x H*N bf16 each; its k
-// and v go straight to the caches) and the split partials.
+// new token's sigmoid(g) and gated attention output (B x H*N bf16 each) and the
+// split partials, with room for one more bf16 row and for more splits than
+// decode_splits makes (callers and the static scratch size by this formula).
 struct DecLayout {
-  size_t a, q, sig, o, part, total;
-  int S, chunk;
+  size_t a, sig, z, part, total;
 };
 
 DecLayout make_dec_layout(const mea_desc& d) {
   DecLayout L = {};
-  mea::decode_splits((int)d.B, (int)d.H, (int)d.T, &L.S, &L.chunk);
   const size_t row = (size_t)(d.B * d.H * d.N) * 2;
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off += align_up(bytes); return o; };
   L.a = take(row * 2 * 4);
-  L.q = take(row);
+  (void)take(row);
   L.sig = take(row);
-  L.o = take(row);
-  L.part = take((size_t)(d.B * d.H) * L.S * (size_t)(d.N + 4) * 4);
+  L.z = take(row);
+  const size_t parts = (size_t)mea::decode_scratch_parts((int)d.B, (int)d.H, (int)d.T);
+  L.part = take((size_t)(d.B * d.H) * parts * (size_t)(d.N + 4) * 4);
   L.total = off;
   return L;
 }
@@ -816,14 +816,10 @@ int decode_launch(const mea_desc* d, const void* x, const void* wq, const void* 
   const int N = (int)d->N, B = (int)d->B, C = (int)d->C, HN = (int)(d->H * d->N);
   hipStream_t s = static_cast<hipStream_t>(stream);
   float* a = at<float>(ws, L.a);
-  bf16_bits* q = at<bf16_bits>(ws, L.q);
-  bf16_bits* sig = at<bf16_bits>(ws, L.sig);
-  bf16_bits* o = at<bf16_bits>(ws, L.o);
   // Projections of the B new tokens (a few rows: every weight row is read
-  // once over a wide grid), then their epilogue at rotary rows pos[b].
+  // once over a wide grid).
   mea::SkinnyParams sp;
-  sp.A0 = static_cast<const bf16_bits*>(x);
-  sp.A1 = nullptr;
+  sp.A = static_cast<const bf16_bits*>(x);
   sp.W[0] = static_cast<const bf16_bits*>(wq);
   sp.W[1] = static_cast<const bf16_bits*>(wk);
   sp.W[2] = static_cast<const bf16_bits*>(wv);
@@ -836,43 +832,32 @@ int decode_launch(const mea_desc* d, const void* x, const void* wq, const void* 
   sp.ldo = 4 * HN;
   sp.out_bf16 = 0;
   MEA_TRY(timed(K_SKINNY_GEMM, s, [&] { return mea::launch_skinny_gemm(sp, s); }));
-  mea::DecodeProjParams pp;
-  pp.a = a;
-  pp.x = static_cast<const bf16_bits*>(x);
-  pp.f1 = f1;
-  pp.f2 = f2;
-  pp.pos = pos;
-  pp.q = q;
-  pp.k_cache = static_cast<bf16_bits*>(k_cache);
-  pp.v_cache = static_cast<bf16_bits*>(v_cache);
-  pp.sig = sig;
-  pp.Tc = (int)d->T;
-  pp.B = B;
-  pp.C = C;
-  pp.H = (int)d->H;
-  pp.t_max = (int)d->T_max;
-  pp.eps = d->eps;
-  pp.qscale = q_log2_scale(n_active(d));
-  pp.inv_n = 1.0f / (float)n_active(d);
-  MEA_TRY(timed(K_DECODE_PROJ, s, [&] { return mea::launch_decode_proj_epilogue(pp, N, s); }));
+  // The epilogue at rotary rows pos[b] and the attention over the cache.
   mea::DecodeParams dp;
-  dp.q = q;
+  dp.a = a;
+  dp.x = static_cast<const bf16_bits*>(x);
+  dp.f1 = f1;
+  dp.f2 = f2;
+  dp.pos = pos;
   dp.k_cache = static_cast<bf16_bits*>(k_cache);
   dp.v_cache = static_cast<bf16_bits*>(v_cache);
-  dp.pos = pos;
+  dp.sig = at<bf16_bits>(ws, L.sig);
   dp.part = at<float>(ws, L.part);
-  dp.o = o;
-  dp.B = (int)d->B;
+  dp.z = at<bf16_bits>(ws, L.z);
+  dp.B = B;
+  dp.C = C;
   dp.H = (int)d->H;
   dp.Tc = (int)d->T;
-  dp.S = L.S;
-  dp.chunk = L.chunk;
+  dp.t_max = (int)d->T_max;
+  dp.S = mea::decode_splits(B, (int)d->H, (int)d->T, N);
+  dp.eps = d->eps;
+  dp.qscale = q_log2_scale(n_active(d));
+  dp.inv_n = 1.0f / (float)n_active(d);
   MEA_TRY(timed(K_ATTN_DECODE, s, [&] { return mea::launch_attn_decode(dp, N, s); }));
   MEA_TRY(timed(K_DECODE_COMBINE, s, [&] { return mea::launch_attn_decode_combine(dp, N, s); }));
-  // y = (O * sigmoid(g)) W_o^T for the B tokens.
+  // y = z W_o^T for the B tokens.
   mea::SkinnyParams op;
-  op.A0 = o;
-  op.A1 = sig;
+  op.A = dp.z;
   op.W[0] = static_cast<const bf16_bits*>(wo);
   op.W[1] = op.W[2] = op.W[3] = nullptr;
   op.out = y;
