@@ -8,7 +8,9 @@ cannot run and every entry point raises.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import functools
 import threading
 from pathlib import Path
 
@@ -133,12 +135,39 @@ def desc(B: int, T: int, C: int, H: int, N: int, T_max: int, eps: float, N_activ
                    int(bool(tables_bf16)))
 
 
+@functools.lru_cache(maxsize=512)
+def plan(B: int, T: int, C: int, H: int, N: int, T_max: int, eps: float, N_active: int, tables_bf16: bool,
+         which: int, T_ws: int) -> tuple[MeaDesc, int]:
+    """The descriptor of a call (the library only reads it) and the workspace
+    bytes of pass ``which`` (mea_workspace_bytes on a descriptor with T_max =
+    T_ws), kept by their values: building both took 5 us of host time a call."""
+    d_ws = desc(B, T, C, H, N, T_ws, eps, N_active, tables_bf16)
+    return desc(B, T, C, H, N, T_max, eps, N_active, tables_bf16), load().mea_workspace_bytes(d_ws, which)
+
+
+@functools.lru_cache(maxsize=512)
+def decode_plan(B: int, T: int, C: int, H: int, N: int, eps: float, N_active: int) -> tuple[MeaDesc, int]:
+    """The same for a decode step against a cache of T rows."""
+    d = desc(B, T, C, H, N, T, eps, N_active)
+    return d, load().mea_decode_workspace_bytes(d)
+
+
+_same_device = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """A context with ``device`` current (nothing to do where it is already)."""
+    return _same_device if torch.cuda.current_device() == device.index else torch.cuda.device(device)
+
+
 def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
 def stream_of(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's handle (without building a Stream object)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def profile_enable(on: bool) -> None:

@@ -54,6 +54,9 @@ MAX_C_BACKWARD = 16384
 MAX_HN_C = 1 << 29  # H * N * C below this: 32-bit element indices into the stacked weights
 
 
+_WEIGHT_NAMES = ("q_proj", "k_proj", "v_proj", "g_proj", "o_proj")
+
+
 def _validate(x, weights, factor1, factor2, H: int, N: int, eps: float, need_backward: bool) -> None:
     if not isinstance(x, torch.Tensor) or x.dim() != 3:
         raise ValueError("x must be a (B, T, C) tensor")
@@ -73,14 +76,15 @@ def _validate(x, weights, factor1, factor2, H: int, N: int, eps: float, need_bac
     HN = H * N
     if HN * C >= MAX_HN_C:
         raise ValueError(f"H*N*C = {HN * C} must be below 2^29")
-    names = ("q_proj", "k_proj", "v_proj", "g_proj", "o_proj")
-    shapes = ((HN, C),) * 4 + ((C, HN),)
-    for name, w, shp in zip(names, weights, shapes):
-        if tuple(w.shape) != shp:
+    dev, shp = x.device, (HN, C)
+    for name, w in zip(_WEIGHT_NAMES, weights):
+        if name == "o_proj":
+            shp = (C, HN)
+        if w.shape != shp:
             raise ValueError(f"{name}.weight has shape {tuple(w.shape)}, expected {shp}")
-        if w.dtype != torch.bfloat16:
+        if w.dtype is not torch.bfloat16:
             raise TypeError(f"{name}.weight must be bfloat16, got {w.dtype}")
-        if w.device != x.device:
+        if w.device != dev:
             raise ValueError(f"{name}.weight is on {w.device}, x is on {x.device}")
     for name, f in (("factor1", factor1), ("factor2", factor2)):
         if f.dim() != 2 or f.shape[1] != N:
@@ -89,7 +93,7 @@ def _validate(x, weights, factor1, factor2, H: int, N: int, eps: float, need_bac
             raise ValueError(f"{name} has {f.shape[0]} rows, fewer than T={T}")
         if f.dtype not in (torch.bfloat16, torch.float16, torch.float32):
             raise TypeError(f"{name} must be a floating tensor, got {f.dtype}")
-        if f.device != x.device:
+        if f.device != dev:
             raise ValueError(f"{name} is on {f.device}, x is on {x.device}")
     if factor1.shape != factor2.shape:
         raise ValueError("factor1 and factor2 must have the same shape")
@@ -133,11 +137,13 @@ def _tables32(factor1: torch.Tensor, factor2: torch.Tensor, T: int):
         N, dev = factor1.shape[1], factor1.device
         out = torch.empty((2, T, N), device=dev, dtype=torch.float32)
         f1, f2 = out[0], out[1]
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = _lib.load().mea_table_rows(factor1.data_ptr(), factor2.data_ptr(), T, N, f1.data_ptr(), f2.data_ptr(),
                                             _lib.stream_of(dev))
         _lib.check(rc, "mea_table_rows")
         return f1, f2
+    if (factor1.dtype == factor2.dtype == torch.float32 and factor1.is_contiguous() and factor2.is_contiguous()):
+        return factor1, factor2  # the library reads the first T rows
     return factor1[:T].float().contiguous(), factor2[:T].float().contiguous()
 
 
@@ -188,16 +194,15 @@ class FusedAttentionFunction(torch.autograd.Function):
         xc = x.contiguous()
         wc = [w.contiguous() for w in weights]
         f1, f2 = _tables32(factor1, factor2, T)
-        d = _lib.desc(B, T, C, H, N, T, eps, n_active, _bf16_tables(factor1, factor2))
+        d, ws_bytes = _lib.plan(B, T, C, H, N, T, eps, n_active, _bf16_tables(factor1, factor2), _lib.MEA_PASS_FWD, T)
         y = torch.empty((B, T, C), device=dev, dtype=torch.bfloat16)
         if need_bwd:
             o_save = torch.empty((B, T, H * N), device=dev, dtype=torch.bfloat16)
             lse = torch.empty((B, H, T), device=dev, dtype=torch.float32)
         else:
             o_save = lse = None
-        ws_bytes = lib.mea_workspace_bytes(d, _lib.MEA_PASS_FWD)
         ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = lib.mea_fwd(
                 d, xc.data_ptr(), *[w.data_ptr() for w in wc], f1.data_ptr(), f2.data_ptr(), y.data_ptr(),
                 _lib.ptr(o_save), _lib.ptr(lse), ws.data_ptr(), ws_bytes, _lib.stream_of(dev),
@@ -217,18 +222,18 @@ class FusedAttentionFunction(torch.autograd.Function):
         B, T, C = x.shape
         dev = x.device
         dy = grad_output.to(torch.bfloat16).contiguous()
-        d = _lib.desc(B, T, C, H, N, T, eps, ctx.n_active, _bf16_tables(factor1, factor2))
+        want_f = ctx.needs_input_grad[6] or ctx.needs_input_grad[7]
+        d, ws_bytes = _lib.plan(B, T, C, H, N, T, eps, ctx.n_active, _bf16_tables(factor1, factor2),
+                                _lib.MEA_PASS_BWD_TABLES if want_f else _lib.MEA_PASS_BWD, T)
         dx = torch.empty_like(x)
         dws = [torch.empty_like(w) for w in (wq, wk, wv, wg, wo)]
-        want_f = ctx.needs_input_grad[6] or ctx.needs_input_grad[7]
         if want_f:
             df1 = torch.empty((T, N), device=dev, dtype=torch.float32)
             df2 = torch.empty((T, N), device=dev, dtype=torch.float32)
         else:
             df1 = df2 = None
-        ws_bytes = lib.mea_workspace_bytes(d, _lib.MEA_PASS_BWD_TABLES if want_f else _lib.MEA_PASS_BWD)
         ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = lib.mea_bwd(
                 d, dy.data_ptr(), x.data_ptr(), wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), wg.data_ptr(),
                 wo.data_ptr(), f1.data_ptr(), f2.data_ptr(), o_save.data_ptr(), lse.data_ptr(), dx.data_ptr(),
@@ -314,17 +319,15 @@ class FusedAttentionVarlenFunction(torch.autograd.Function):
         cu = cu_seqlens.contiguous()
         f1, f2 = _tables32(factor1, factor2, max_len)
         tb16 = _bf16_tables(factor1, factor2)
-        d = _lib.desc(1, total, C, H, N, max_len, eps, n_active, tb16)
-        d_ws = _lib.desc(1, total, C, H, N, total, eps, n_active, tb16)
+        d, ws_bytes = _lib.plan(1, total, C, H, N, max_len, eps, n_active, tb16, _lib.MEA_PASS_FWD, total)
         y = torch.empty((total, C), device=dev, dtype=torch.bfloat16)
         if need_bwd:
             o_save = torch.empty((total, H * N), device=dev, dtype=torch.bfloat16)
             lse = torch.empty((H, total), device=dev, dtype=torch.float32)
         else:
             o_save = lse = None
-        ws_bytes = lib.mea_workspace_bytes(d_ws, _lib.MEA_PASS_FWD)
         ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = lib.mea_fwd_varlen(
                 d, cu.data_ptr(), nseq, max_len, xc.data_ptr(), *[w.data_ptr() for w in wc], f1.data_ptr(),
                 f2.data_ptr(), y.data_ptr(), _lib.ptr(o_save), _lib.ptr(lse), ws.data_ptr(), ws_bytes,
@@ -348,19 +351,18 @@ class FusedAttentionVarlenFunction(torch.autograd.Function):
         nseq = cu.numel() - 1
         dy = grad_output.to(torch.bfloat16).contiguous()
         tb16 = _bf16_tables(factor1, factor2)
-        d = _lib.desc(1, total, C, H, N, max_len, eps, ctx.n_active, tb16)
-        d_ws = _lib.desc(1, total, C, H, N, total, eps, ctx.n_active, tb16)
+        want_f = ctx.needs_input_grad[6] or ctx.needs_input_grad[7]
+        d, ws_bytes = _lib.plan(1, total, C, H, N, max_len, eps, ctx.n_active, tb16,
+                                _lib.MEA_PASS_BWD_TABLES if want_f else _lib.MEA_PASS_BWD, total)
         dx = torch.empty_like(x)
         dws = [torch.empty_like(w) for w in (wq, wk, wv, wg, wo)]
-        want_f = ctx.needs_input_grad[6] or ctx.needs_input_grad[7]
         if want_f:
             df1 = torch.empty((max_len, N), device=dev, dtype=torch.float32)
             df2 = torch.empty((max_len, N), device=dev, dtype=torch.float32)
         else:
             df1 = df2 = None
-        ws_bytes = lib.mea_workspace_bytes(d_ws, _lib.MEA_PASS_BWD_TABLES if want_f else _lib.MEA_PASS_BWD)
         ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = lib.mea_bwd_varlen(
                 d, cu.data_ptr(), nseq, max_len, dy.data_ptr(), x.data_ptr(), wq.data_ptr(), wk.data_ptr(),
                 wv.data_ptr(), wg.data_ptr(), wo.data_ptr(), f1.data_ptr(), f2.data_ptr(), o_save.data_ptr(),

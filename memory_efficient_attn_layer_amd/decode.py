@@ -104,11 +104,10 @@ def prefill(x, q_weight, k_weight, v_weight, g_weight, o_weight, factor1, factor
     wc = [w.contiguous() for w in weights]
     tb16 = factor1.dtype == torch.bfloat16 and factor2.dtype == torch.bfloat16
     f1, f2 = _tables(factor1, factor2, Tc)
-    d = _lib.desc(B, T, C, H, N, Tc, eps, n_active, tb16)
+    d, ws_bytes = _lib.plan(B, T, C, H, N, Tc, eps, n_active, tb16, _lib.MEA_PASS_FWD, Tc)
     y = torch.empty((B, T, C), device=dev, dtype=torch.bfloat16)
-    ws_bytes = lib.mea_workspace_bytes(d, _lib.MEA_PASS_FWD)
     ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = lib.mea_prefill(d, xc.data_ptr(), *[w.data_ptr() for w in wc], f1.data_ptr(), f2.data_ptr(),
                              y.data_ptr(), cache.k.data_ptr(), cache.v.data_ptr(), Tc, ws.data_ptr(), ws_bytes,
                              _lib.stream_of(dev))
@@ -150,13 +149,12 @@ def _decode_launch(x3, weights, factor1, factor2, H, N, n_active, pos, cache, ep
     wc = [w.contiguous() for w in weights]
     posc = pos.contiguous()
     f1, f2 = _tables(factor1, factor2, Tc)
-    d = _lib.desc(B, Tc, C, H, N, Tc, eps, n_active)
+    d, ws_bytes = _lib.decode_plan(B, Tc, C, H, N, eps, n_active)
     y = torch.empty((B, 1, C), device=dev, dtype=torch.bfloat16)
-    ws_bytes = lib.mea_decode_workspace_bytes(d)
     if ws_bytes == 0:
         raise ValueError("unsupported decode shape")
     ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = lib.mea_decode(d, xc.data_ptr(), *[w.data_ptr() for w in wc], f1.data_ptr(), f2.data_ptr(),
                             posc.data_ptr(), cache.k.data_ptr(), cache.v.data_ptr(), y.data_ptr(), ws.data_ptr(),
                             ws_bytes, _lib.stream_of(dev))
