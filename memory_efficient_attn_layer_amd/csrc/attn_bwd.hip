@@ -167,8 +167,11 @@ __device__ __forceinline__ void head_row_bwd(const float* stg, int FP, int t0, c
 // their exact bf16 terms against (1, 1, 1) selectors; the LDS start values
 // save those MFMAs: dQ -0.9%, dK/dV -3%.)
 // ---------------------------------------------------------------------------
-template <int N, bool VARLEN>
-__global__ __launch_bounds__(256, N <= 64 ? 3 : N == 256 ? 1 : 2) void attn_bwd_dq_kernel(AttnBwdParams p) {
+// SPLIT: wave groups of four that share the block's queries and take its key
+// tiles in turn, as in the forward.
+template <int N, bool VARLEN, int SPLIT = 1>
+__global__ __launch_bounds__(256 * SPLIT, SPLIT > 1 ? 1 : N <= 64 ? 3 : N == 256 ? 1 : 2) void attn_bwd_dq_kernel(
+    AttnBwdParams p) {
   constexpr int QW = 32;                 // queries per wave
   constexpr int QB = QW / 32;            // 32-query MFMA blocks per wave
   constexpr int BQ = 4 * QW;             // queries per workgroup
@@ -180,9 +183,12 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 256 ? 1 : 2) void attn_bwd_
   constexpr int SM_LOOP = 4 * TILE * 2;  // bytes: [stage][K | V]
   constexpr int SM_STAT = 4 * QB * 2 * 4 * 32 * 16;  // bytes: [wave][qb][lse | delta][copy][query] x 4
   constexpr int SM_OUT = 4 * QW * FP * 4;
-  constexpr int SMEM = SM_LOOP + SM_STAT > SM_OUT ? SM_LOOP + SM_STAT : SM_OUT;
+  // The groups' tiles, the statistics of the queries (the same for each group).
+  constexpr int SMEM = SPLIT * SM_LOOP + SM_STAT > SM_OUT ? SPLIT * SM_LOOP + SM_STAT : SM_OUT;
+  static_assert(SPLIT <= 2, "one exchange of partial gradients");
   __shared__ __attribute__((aligned(16))) unsigned char smem_raw[SMEM];
-  bf16_bits* smem = reinterpret_cast<bf16_bits*>(smem_raw);
+  const int grp = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  bf16_bits* smem = reinterpret_cast<bf16_bits*>(smem_raw + grp * SM_LOOP);
 
   // Each XCD walks whole heads (heaviest query block first), so the K/V
   // tiles of a head are fetched once into that XCD's L2. VARLEN: packed
@@ -193,7 +199,7 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 256 ? 1 : 2) void attn_bwd_
   if constexpr (!VARLEN) {
     T = p.T;
     const int nqb = (T + BQ - 1) / BQ;
-    const int lid = attn_item(blockIdx.x, p.B * nh * nqb, nqb, N <= 64 ? 3 : 1);
+    const int lid = attn_item(blockIdx.x, p.B * nh * nqb, nqb, N <= 64 && SPLIT == 1 ? 3 : 1);
     const int bh = lid / nqb;
     qi = nqb - 1 - lid % nqb;
     b = bh / nh;
@@ -203,7 +209,7 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 256 ? 1 : 2) void attn_bwd_
     tok_row0 = (size_t)b * T;
   } else {
     const int nqb = (p.max_len + BQ - 1) / BQ;
-    const int lid = attn_item(blockIdx.x, p.nseq * nh * nqb, nqb, N <= 64 ? 3 : 1);
+    const int lid = attn_item(blockIdx.x, p.nseq * nh * nqb, nqb, N <= 64 && SPLIT == 1 ? 3 : 1);
     const int bh = lid / nqb;
     qi = nqb - 1 - lid % nqb;
     b = bh / nh;
@@ -220,7 +226,7 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 256 ? 1 : 2) void attn_bwd_
     const int hd = h_first;
     const size_t head_row0 = hrow_base + (size_t)hd * hrow_step;
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(SPLIT == 1 ? tid >> 6 : (tid >> 6) & 3);
     const int c = lane & 31, h = lane >> 5;
     const int q0w = qi * BQ + wave * QW;
     const int kv_end = min(T, qi * BQ + BQ);
@@ -236,7 +242,7 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 256 ? 1 : 2) void attn_bwd_
     // the four reads that fill an accumulator from being merged into one read
     // and twelve register moves.
     bf16x8 qf[QB][KS], df[QB][KS];
-    f32x4* statq = reinterpret_cast<f32x4*>(smem_raw + SM_LOOP) + wave * QB * 256;
+    f32x4* statq = reinterpret_cast<f32x4*>(smem_raw + SPLIT * SM_LOOP) + wave * QB * 256;
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       const int t = min(q0w + 32 * qb + c, T - 1);
@@ -383,6 +389,34 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 256 ? 1 : 2) void attn_bwd_
     // inside the sequence; the split point is per wave (one barrier per tile
     // in either loop keeps the waves in step).
     const int nfull = min(nkv, min(q0w + 1, T) / BKV);
+    if constexpr (SPLIT > 1) {
+      // (Both groups write the same statistics; each wave reads its own
+      // queries' after the first barrier.)
+      if (grp < nkv) issue_tile(grp * BKV, 0);
+      wait_vmcnt0();
+      __syncthreads();
+      int j = grp, s = 0;  // tile, LDS stage
+      for (; j < nfull; j += SPLIT, s ^= 1) {
+        if (j + SPLIT < nkv) issue_tile((j + SPLIT) * BKV, s ^ 1);
+        const bf16_bits* ks_t = smem + s * 2 * TILE;
+        step(ks_t, ks_t + TILE, 0, j * BKV, std::false_type{});
+        step(ks_t, ks_t + TILE, 1, j * BKV + 32, std::false_type{});
+        wait_vmcnt0();
+        __syncthreads();
+      }
+      for (; j < nkv; j += SPLIT, s ^= 1) {
+        if (j + SPLIT < nkv) issue_tile((j + SPLIT) * BKV, s ^ 1);
+        const bf16_bits* ks_t = smem + s * 2 * TILE;
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+          const int kb0 = j * BKV + st * 32;
+          if (kb0 <= q0w + QW - 1) step(ks_t, ks_t + TILE, st, kb0, std::true_type{});
+        }
+        wait_vmcnt0();
+        __syncthreads();
+      }
+      if (j - grp < nkv) __syncthreads();  // every group passes the same barriers
+    } else {
     issue_tile(0, 0);
     wait_vmcnt0();  // also retires the q/dO fragment loads
     __syncthreads();
@@ -406,20 +440,37 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 256 ? 1 : 2) void attn_bwd_
       wait_vmcnt0();
       __syncthreads();
     }
+    }
 
-    // Stage dQ (times the softmax scale) as fp32 rows, then the q chain.
+    // Stage dQ (times the softmax scale) as fp32 rows, then the q chain. With
+    // two groups group 1 stages its share and group 0 adds its own to it.
     float* stg = reinterpret_cast<float*>(smem_raw) + wave * QW * FP;
+    auto stage = [&](auto add_tag) {
 #pragma unroll
-    for (int qb = 0; qb < QB; ++qb)
+      for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
-      for (int db = 0; db < DB; ++db)
+        for (int db = 0; db < DB; ++db)
 #pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-          const f32x16& a = dq[qb][db];
-          const f32x4 v = {a[4 * r4], a[4 * r4 + 1], a[4 * r4 + 2], a[4 * r4 + 3]};
-          *reinterpret_cast<f32x4*>(stg + (32 * qb + c) * FP + 32 * db + 8 * r4 + 4 * h) = v * p.scale;
-        }
-    __syncthreads();
+          for (int r4 = 0; r4 < 4; ++r4) {
+            const f32x16& a = dq[qb][db];
+            const f32x4 v = {a[4 * r4], a[4 * r4 + 1], a[4 * r4 + 2], a[4 * r4 + 3]};
+            f32x4* at = reinterpret_cast<f32x4*>(stg + (32 * qb + c) * FP + 32 * db + 8 * r4 + 4 * h);
+            if (decltype(add_tag)::value)
+              *at += v * p.scale;
+            else
+              *at = v * p.scale;
+          }
+    };
+    if constexpr (SPLIT > 1) {
+      if (grp == 1) stage(std::false_type{});
+      __syncthreads();
+      if (grp == 0) stage(std::true_type{});
+      __syncthreads();
+      if (grp == 1) return;
+    } else {
+      stage(std::false_type{});
+      __syncthreads();
+    }
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb)
       head_row_bwd<N>(stg + 32 * qb * FP, FP, q0w + 32 * qb, p, T, tok_row0, head_row0, true, p.q,
@@ -454,8 +505,12 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 256 ? 1 : 2) void attn_bwd_
 // gradients, whose extra state would spill at 256 registers) runs one wave
 // per SIMD.
 // ---------------------------------------------------------------------------
-template <int N, bool VARLEN>
-__global__ __launch_bounds__(256, N <= 64 ? 3 : N == 128 ? 2 : 1) void attn_bwd_dkdv_kernel(AttnBwdParams p) {
+// SPLIT: wave groups of four that share the block's keys and take its query
+// tiles in turn; at the end each group takes the other's share of one of the two
+// gradients and runs that row tail.
+template <int N, bool VARLEN, int SPLIT = 1>
+__global__ __launch_bounds__(256 * SPLIT, SPLIT > 1 ? 1 : N <= 64 ? 3 : N == 128 ? 2 : 1) void attn_bwd_dkdv_kernel(
+    AttnBwdParams p) {
   constexpr int KW = 32;                 // keys per wave
   constexpr int KB = KW / 32;            // 32-key MFMA blocks per wave
   static_assert(KB == 1, "one 32-key block per wave");
@@ -469,13 +524,18 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 128 ? 2 : 1) void attn_bwd_
   constexpr int SM_LOOP = 2 * 2 * TILE * 2 + 2 * 2 * BQ * 4;  // bytes
   constexpr int SM_V = 4 * KS * 64 * 16;  // bytes: each wave's V^T fragments, [wave][ks][lane]
   constexpr int SM_OUT = 4 * 32 * FP * 4;
-  constexpr int SMEM = SM_LOOP + SM_V > SM_OUT ? SM_LOOP + SM_V : SM_OUT;
+  // The groups' tiles and statistics, the V fragments (the same for each
+  // group); then the staged rows of one gradient per group.
+  constexpr int SM_MAIN = SPLIT * SM_LOOP + SM_V;
+  constexpr int SMEM = SM_MAIN > SPLIT * SM_OUT ? SM_MAIN : SPLIT * SM_OUT;
+  static_assert(SPLIT <= 2, "one exchange of partial gradients");
   __shared__ __attribute__((aligned(16))) unsigned char smem[SMEM];
-  bf16_bits* tiles = reinterpret_cast<bf16_bits*>(smem);           // [stage][Q | dO]
+  const int grp = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  bf16_bits* tiles = reinterpret_cast<bf16_bits*>(smem + grp * SM_LOOP);  // [stage][Q | dO]
   // [stage][-lse*log2e | -delta][query]: the accumulator start values of the
   // tile's queries.
-  float* statf = reinterpret_cast<float*>(smem + 2 * 2 * TILE * 2);
-  u32x4* vown = reinterpret_cast<u32x4*>(smem + SM_LOOP);
+  float* statf = reinterpret_cast<float*>(smem + grp * SM_LOOP + 2 * 2 * TILE * 2);
+  u32x4* vown = reinterpret_cast<u32x4*>(smem + SPLIT * SM_LOOP);
 
   // Each XCD walks whole heads, the key block that sees the most queries
   // first, so the Q/dO tiles of a head are shared in one L2. VARLEN: packed
@@ -486,7 +546,7 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 128 ? 2 : 1) void attn_bwd_
   if constexpr (!VARLEN) {
     T = p.T;
     const int nkb = (T + BKV - 1) / BKV;
-    const int lid = attn_item(blockIdx.x, p.B * nh * nkb, nkb, N <= 64 ? 3 : 1);
+    const int lid = attn_item(blockIdx.x, p.B * nh * nkb, nkb, N <= 64 && SPLIT == 1 ? 3 : 1);
     const int bh = lid / nkb;
     ki = lid % nkb;
     b = bh / nh;
@@ -496,7 +556,7 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 128 ? 2 : 1) void attn_bwd_
     tok_row0 = (size_t)b * T;
   } else {
     const int nkb = (p.max_len + BKV - 1) / BKV;
-    const int lid = attn_item(blockIdx.x, p.nseq * nh * nkb, nkb, N <= 64 ? 3 : 1);
+    const int lid = attn_item(blockIdx.x, p.nseq * nh * nkb, nkb, N <= 64 && SPLIT == 1 ? 3 : 1);
     const int bh = lid / nkb;
     ki = lid % nkb;
     b = bh / nh;
@@ -512,7 +572,7 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 128 ? 2 : 1) void attn_bwd_
   {
     const int hd = h_first;
     const size_t head_row0 = hrow_base + (size_t)hd * hrow_step;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = SPLIT == 1 ? threadIdx.x : threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
     const int c = lane & 31, h = lane >> 5;
     const int k0 = ki * BKV, kw0 = k0 + wave * KW;
     const size_t head_off = head_row0 * N;
@@ -603,9 +663,9 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 128 ? 2 : 1) void attn_bwd_
     // there are key blocks), which cut this kernel's HBM reads from 2.74 to
     // 2.27 GB per launch at B64 T4096 C512 H8 N64.
     const int nq = (T - k0 + BQ - 1) / BQ;
-    issue_tile(k0 + (nq - 1) * BQ, 0);
+    if (SPLIT == 1 || grp < nq) issue_tile(k0 + (nq - 1 - grp) * BQ, 0);
     wait_vmcnt0();
-    publish_stats(0);
+    if (SPLIT == 1 || grp < nq) publish_stats(0);
     __syncthreads();
     // One query tile. MASKED: the tile may touch the causal diagonal or the
     // sequence end (per-step tests and masks); the tiles between hold only
@@ -613,10 +673,11 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 128 ? 2 : 1) void attn_bwd_
     auto tile = [&](int it, auto masked_tag) {
       constexpr bool MASKED = decltype(masked_tag)::value;
       const int q0 = k0 + (nq - 1 - it) * BQ;
-      if (it + 1 < nq) issue_tile(q0 - BQ, (it + 1) & 1);
-      const bf16_bits* qt = tiles + (it & 1) * 2 * TILE;
+      const int tr = it / SPLIT;  // this group's turn
+      if (it + SPLIT < nq) issue_tile(q0 - SPLIT * BQ, (tr + 1) & 1);
+      const bf16_bits* qt = tiles + (tr & 1) * 2 * TILE;
       const bf16_bits* dt = qt + TILE;
-      const float* stf = statf + (it & 1) * 2 * BQ;
+      const float* stf = statf + (tr & 1) * 2 * BQ;
       // One 32-query step in three parts: S and dP (MFMA), P and dS (exp2,
       // multiply, convert; DIAG steps also mask key > query and query >= T),
       // then the dV and dK updates (MFMA).
@@ -700,20 +761,65 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 128 ? 2 : 1) void attn_bwd_
         if (!MASKED) __builtin_amdgcn_sched_barrier(0);
       }
       wait_vmcnt0();
-      if (it + 1 < nq) publish_stats((it + 1) & 1);
+      if (it + SPLIT < nq) publish_stats((tr + 1) & 1);
       __syncthreads();
     };
     // Tiles it < nfull lie wholly above the block's keys (q0 >= k0 + BKV);
     // the first one (the highest queries) may run past the sequence end.
     const int nfull = nq - BKV / BQ;
+    if constexpr (SPLIT > 1) {
+      int it = grp;
+      if (grp == 0 && nfull > 0 && (T - k0) % BQ != 0) {
+        tile(it, std::true_type{});
+        it += SPLIT;
+      }
+      for (; it < nfull; it += SPLIT) tile(it, std::false_type{});
+      for (; it < nq; it += SPLIT) tile(it, std::true_type{});
+      if (it - grp < nq) __syncthreads();  // every group passes the same barriers
+    } else {
     int it = 0;
     if (nfull > 0 && (T - k0) % BQ != 0) tile(it++, std::true_type{});
     for (; it < nfull; ++it) tile(it, std::false_type{});
     for (; it < nq; ++it) tile(it, std::true_type{});
+    }
 
     // Epilogue per 32-key block: stage dV (then dK * scale) as fp32 rows and run
     // the row-wise tails (rx scale; k RMSNorm + rotary backward for dK).
     float* stg = reinterpret_cast<float*>(smem) + wave * 32 * FP;
+    if constexpr (SPLIT > 1) {
+      // Group 1 stages its dV and group 0 its dK (in the second area); each adds
+      // its own share to the other's rows and runs that tail.
+      float* stg_k = stg + 4 * 32 * FP;
+      auto stage = [&](float* at, const f32x16 (&g)[DB], float scale, auto add_tag) {
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int r4 = 0; r4 < 4; ++r4) {
+            const f32x4 v = {g[db][4 * r4], g[db][4 * r4 + 1], g[db][4 * r4 + 2], g[db][4 * r4 + 3]};
+            f32x4* w = reinterpret_cast<f32x4*>(at + c * FP + 32 * db + 8 * r4 + 4 * h);
+            if (decltype(add_tag)::value)
+              *w += v * scale;
+            else
+              *w = v * scale;
+          }
+      };
+      const float ks = p.scale / p.qscale;
+      if (grp == 0)
+        stage(stg_k, dk[0], ks, std::false_type{});
+      else
+        stage(stg, dv[0], 1.0f, std::false_type{});
+      __syncthreads();
+      if (grp == 0)
+        stage(stg, dv[0], 1.0f, std::true_type{});
+      else
+        stage(stg_k, dk[0], ks, std::true_type{});
+      __syncthreads();
+      if (grp == 0)
+        head_row_bwd<N>(stg, FP, kw0, p, T, tok_row0, head_row0, false, nullptr, 1.0f, nullptr, p.dav, nullptr);
+      else
+        head_row_bwd<N>(stg_k, FP, kw0, p, T, tok_row0, head_row0, true, p.k, 1.0f, p.rk, p.dak, p.dotk);
+      return;
+    }
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
 #pragma unroll
@@ -744,12 +850,24 @@ __global__ __launch_bounds__(256, N <= 64 ? 3 : N == 128 ? 2 : 1) void attn_bwd_
 template <int N, bool VAR>
 struct DqKernel {
   static void launch(const AttnBwdParams& p, int G, hipStream_t s) {
+    if constexpr (N <= 128) {
+      if (attn_split(G, VAR ? p.max_len : p.T, N)) {
+        hipLaunchKernelGGL((attn_bwd_dq_kernel<N, VAR, 2>), dim3(G), dim3(512), 0, s, p);
+        return;
+      }
+    }
     hipLaunchKernelGGL((attn_bwd_dq_kernel<N, VAR>), dim3(G), dim3(256), 0, s, p);
   }
 };
 template <int N, bool VAR>
 struct DkdvKernel {
   static void launch(const AttnBwdParams& p, int G, hipStream_t s) {
+    if constexpr (N <= 128) {
+      if (attn_split(G, VAR ? p.max_len : p.T, N)) {
+        hipLaunchKernelGGL((attn_bwd_dkdv_kernel<N, VAR, 2>), dim3(G), dim3(512), 0, s, p);
+        return;
+      }
+    }
     hipLaunchKernelGGL((attn_bwd_dkdv_kernel<N, VAR>), dim3(G), dim3(256), 0, s, p);
   }
 };

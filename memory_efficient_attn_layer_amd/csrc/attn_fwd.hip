@@ -46,8 +46,13 @@ namespace mea {
 // VARLEN: packed sequences (p.cu); a workgroup's (b, h, query block) becomes
 // (sequence, h, query block) and every row index is taken relative to the
 // sequence's first token.
-template <int N, bool VARLEN>
-__global__ __launch_bounds__(256, N <= 64 ? 4 : N == 128 ? 3 : 1) void attn_fwd_kernel(AttnFwdParams p) {
+// SPLIT: wave groups of four that share the block's queries and take its key
+// tiles in turn, each with LDS tiles of its own; their sums meet in LDS at the
+// end. Two groups run where the grid gives a CU at most one workgroup (see
+// kSplitGrid): a lone wave per SIMD waits out its own S -> exp2 -> PV chain.
+template <int N, bool VARLEN, int SPLIT = 1>
+__global__ __launch_bounds__(256 * SPLIT, SPLIT > 1 ? 1 : N <= 64 ? 4 : N == 128 ? 3 : 1) void attn_fwd_kernel(
+    AttnFwdParams p) {
   constexpr int QW = 32;  // queries per wave
   constexpr int QB = QW / 32;            // 32-query MFMA blocks per wave
   constexpr int BQ = 4 * QW;             // queries per workgroup
@@ -59,8 +64,13 @@ __global__ __launch_bounds__(256, N <= 64 ? 4 : N == 128 ? 3 : 1) void attn_fwd_
   constexpr int LOADS = TILE / 8 / 256;  // 16-byte loads per thread per tile
   constexpr float TAU = 8.f;
   constexpr int OP = N + 8;              // output staging pitch
-  constexpr int SMEM = 4 * TILE > 4 * QW * OP ? 4 * TILE : 4 * QW * OP;
-  __shared__ __attribute__((aligned(16))) bf16_bits smem[SMEM];  // [stage][K | V], then output staging
+  constexpr int SMEM1 = 4 * TILE > 4 * QW * OP ? 4 * TILE : 4 * QW * OP;
+  constexpr int SX = 4 * DB * 16 * 64 * 2;  // fp32 partial outputs of one group (elements of smem)
+  constexpr int SMEM = SPLIT * SMEM1 > (SPLIT - 1) * SX ? SPLIT * SMEM1 : (SPLIT - 1) * SX;
+  static_assert(SPLIT <= 2, "one exchange of partial outputs");
+  // [group][stage][K | V], then the partial outputs, then output staging
+  __shared__ __attribute__((aligned(16))) bf16_bits smem_all[SMEM];
+  __shared__ float sx_ml[SPLIT > 1 ? 2 : 1][SPLIT > 1 ? 256 : 1];
 
   // Each XCD walks whole heads (heaviest query block of a head first), so
   // the K/V tiles of a head are fetched once into that XCD's L2.
@@ -69,7 +79,7 @@ __global__ __launch_bounds__(256, N <= 64 ? 4 : N == 128 ? 3 : 1) void attn_fwd_
   if constexpr (!VARLEN) {
     T = p.T;
     const int nqb = (T + BQ - 1) / BQ;
-    const int lid = attn_item(blockIdx.x, p.B * p.H * nqb, nqb, N <= 64 ? 3 : 1);
+    const int lid = attn_item(blockIdx.x, p.B * p.H * nqb, nqb, N <= 64 && SPLIT == 1 ? 3 : 1);
     bh = lid / nqb;
     qi = nqb - 1 - lid % nqb;
     b = bh / p.H;
@@ -78,7 +88,7 @@ __global__ __launch_bounds__(256, N <= 64 ? 4 : N == 128 ? 3 : 1) void attn_fwd_
     tok_row0 = (size_t)b * T;
   } else {
     const int nqb = (p.max_len + BQ - 1) / BQ;
-    const int lid = attn_item(blockIdx.x, p.nseq * p.H * nqb, nqb, N <= 64 ? 3 : 1);
+    const int lid = attn_item(blockIdx.x, p.nseq * p.H * nqb, nqb, N <= 64 && SPLIT == 1 ? 3 : 1);
     bh = lid / nqb;  // sequence-major (s, h)
     qi = nqb - 1 - lid % nqb;
     b = bh / p.H;
@@ -91,7 +101,9 @@ __global__ __launch_bounds__(256, N <= 64 ? 4 : N == 128 ? 3 : 1) void attn_fwd_
     if (qi * BQ >= T) return;  // past this sequence's end: uniform, before any barrier
   }
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+  const int wave = __builtin_amdgcn_readfirstlane(SPLIT == 1 ? tid >> 6 : (tid >> 6) & 3);
+  bf16_bits* smem = smem_all + grp * SMEM1;
   const int c = lane & 31, h = lane >> 5;
   const int q0w = qi * BQ + wave * QW;
   const int kv_end = min(T, qi * BQ + BQ);
@@ -246,13 +258,14 @@ __global__ __launch_bounds__(256, N <= 64 ? 4 : N == 128 ? 3 : 1) void attn_fwd_
         const bool up = ms > m_i[qb] + TAU;
         if (__any(up)) {
           const float mn = up ? ms : m_i[qb];
-          const float alpha = fast_exp2(m_i[qb] - mn);
+          // (A group's rows may have met no key yet: m_i = -inf.)
+          const float alpha = SPLIT > 1 && !up ? 1.f : fast_exp2(m_i[qb] - mn);
           l_i[qb] *= alpha;
 #pragma unroll
           for (int db = 0; db < DB; ++db) o[qb][db] *= alpha;
           m_i[qb] = mn;
         }
-        const float nm = -m_i[qb];
+        const float nm = SPLIT > 1 && m_i[qb] == -INFINITY ? 0.f : -m_i[qb];
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const float e = fast_exp2(__builtin_fmaf(s[i], p.sl2e, nm));
@@ -293,6 +306,34 @@ __global__ __launch_bounds__(256, N <= 64 ? 4 : N == 128 ? 3 : 1) void attn_fwd_
   auto main_loop = [&](auto fixed_tag) {
     const int nkv = (kv_end + BKV - 1) / BKV;
     const int nfull = min(nkv, min(q0w + 1, T) / BKV);
+    if constexpr (SPLIT > 1) {
+      // Tiles grp, grp + SPLIT, ... of this group.
+      if (grp < nkv) issue_tile(grp * BKV, 0);
+      wait_vmcnt0();
+      __syncthreads();
+      int j = grp, s = 0;  // tile, LDS stage
+      for (; j < nfull; j += SPLIT, s ^= 1) {
+        if (j + SPLIT < nkv) issue_tile((j + SPLIT) * BKV, s ^ 1);
+        const bf16_bits* ks_t = smem + s * 2 * TILE;
+#pragma unroll
+        for (int st = 0; st < BKV / 32; ++st) step(ks_t, ks_t + TILE, st, j * BKV + 32 * st, fixed_tag, std::false_type{});
+        wait_vmcnt0();
+        __syncthreads();
+      }
+      for (; j < nkv; j += SPLIT, s ^= 1) {
+        if (j + SPLIT < nkv) issue_tile((j + SPLIT) * BKV, s ^ 1);
+        const bf16_bits* ks_t = smem + s * 2 * TILE;
+#pragma unroll
+        for (int st = 0; st < BKV / 32; ++st) {
+          const int kb0 = j * BKV + st * 32;
+          if (kb0 <= q0w + QW - 1) step(ks_t, ks_t + TILE, st, kb0, fixed_tag, std::true_type{});
+        }
+        wait_vmcnt0();
+        __syncthreads();
+      }
+      if (j - grp < nkv) __syncthreads();  // every group passes the same barriers
+      return;
+    }
     issue_tile(0, 0);
     wait_vmcnt0();  // also retires the Q fragment loads
     __syncthreads();
@@ -330,6 +371,44 @@ __global__ __launch_bounds__(256, N <= 64 ? 4 : N == 128 ? 3 : 1) void attn_fwd_
     }
   } else {
     main_loop(std::false_type{});
+  }
+
+  if constexpr (SPLIT > 1) {
+    // Group 1's sums (its own maximum each; 0 in the fixed form) join group 0's,
+    // lane for lane. Group 0 holds tile 0, so its maximum is finite.
+    static_assert(QB == 1, "one query block per wave");
+    f32x4* sx = reinterpret_cast<f32x4*>(smem_all) + (size_t)wave * DB * 4 * 64 + lane;
+    const int me = wave * 64 + lane;
+    if (grp == 1) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4)
+          sx[(db * 4 + r4) * 64] = f32x4{o[0][db][4 * r4], o[0][db][4 * r4 + 1], o[0][db][4 * r4 + 2], o[0][db][4 * r4 + 3]};
+      sx_ml[0][SPLIT > 1 ? me : 0] = m_i[0];
+      sx_ml[SPLIT > 1 ? 1 : 0][SPLIT > 1 ? me : 0] = l_i[0];
+    }
+    __syncthreads();
+    if (grp == 0) {
+      const float m1 = sx_ml[0][SPLIT > 1 ? me : 0], l1 = sx_ml[SPLIT > 1 ? 1 : 0][SPLIT > 1 ? me : 0];
+      const float m = fmaxf(m_i[0], m1), a0 = fast_exp2(m_i[0] - m), a1 = fast_exp2(m1 - m);
+      m_i[0] = m;
+      l_i[0] = l_i[0] * a0 + l1 * a1;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+          const f32x4 v = sx[(db * 4 + r4) * 64];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[0][db][4 * r4 + e] = o[0][db][4 * r4 + e] * a0 + v[e] * a1;
+        }
+    }
+    __syncthreads();  // the exchange becomes the staging area
+    if (grp == 1) {
+      __syncthreads();  // the staging barrier below
+      return;
+    }
+    smem = smem_all;
   }
 
   // The output gate's rows are requested before the staging that they wait
@@ -378,26 +457,29 @@ __global__ __launch_bounds__(256, N <= 64 ? 4 : N == 128 ? 3 : 1) void attn_fwd_
   }
 }
 
+template <int N, bool VAR>
+static void launch_fwd(const AttnFwdParams& p, int G, hipStream_t s) {
+  if constexpr (N <= 128) {
+    if (attn_split(G, VAR ? p.max_len : p.T, N)) {
+      hipLaunchKernelGGL((attn_fwd_kernel<N, VAR, 2>), dim3(G), dim3(512), 0, s, p);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((attn_fwd_kernel<N, VAR>), dim3(G), dim3(256), 0, s, p);
+}
+
 hipError_t launch_attn_fwd(const AttnFwdParams& p, int N, hipStream_t s) {
   const int BQ = 128;
   const bool var = p.cu != nullptr;
   const int G = var ? p.nseq * p.H * ((p.max_len + BQ - 1) / BQ) : p.B * p.H * ((p.T + BQ - 1) / BQ);
-  if (N == 32 && !var)
-    hipLaunchKernelGGL((attn_fwd_kernel<32, false>), dim3(G), dim3(256), 0, s, p);
-  else if (N == 32)
-    hipLaunchKernelGGL((attn_fwd_kernel<32, true>), dim3(G), dim3(256), 0, s, p);
-  else if (N == 64 && !var)
-    hipLaunchKernelGGL((attn_fwd_kernel<64, false>), dim3(G), dim3(256), 0, s, p);
+  if (N == 32)
+    var ? launch_fwd<32, true>(p, G, s) : launch_fwd<32, false>(p, G, s);
   else if (N == 64)
-    hipLaunchKernelGGL((attn_fwd_kernel<64, true>), dim3(G), dim3(256), 0, s, p);
-  else if (N == 128 && !var)
-    hipLaunchKernelGGL((attn_fwd_kernel<128, false>), dim3(G), dim3(256), 0, s, p);
+    var ? launch_fwd<64, true>(p, G, s) : launch_fwd<64, false>(p, G, s);
   else if (N == 128)
-    hipLaunchKernelGGL((attn_fwd_kernel<128, true>), dim3(G), dim3(256), 0, s, p);
-  else if (N == 256 && !var)
-    hipLaunchKernelGGL((attn_fwd_kernel<256, false>), dim3(G), dim3(256), 0, s, p);
+    var ? launch_fwd<128, true>(p, G, s) : launch_fwd<128, false>(p, G, s);
   else if (N == 256)
-    hipLaunchKernelGGL((attn_fwd_kernel<256, true>), dim3(G), dim3(256), 0, s, p);
+    var ? launch_fwd<256, true>(p, G, s) : launch_fwd<256, false>(p, G, s);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();

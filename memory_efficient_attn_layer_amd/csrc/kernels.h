@@ -93,6 +93,20 @@ struct AttnFwdParams {
   int nseq, max_len;
 };
 constexpr float kFixedBound = 60.0f;
+// Whether the attention kernels run two wave groups per workgroup (SPLIT). A
+// grid below one workgroup per CU is bound by the serial chain of its longest
+// workgroup (load, QK, softmax, PV per tile), so halving that chain pays.
+// Forward / dQ / dK,dV, one group -> two (us): N = 64 with 128 workgroups
+// (T 1024) 33 / 33 / 48 -> 24 / 28 / 35; N = 128 with 96 (B1 T768 H16)
+// 25 / 28 / 38 -> 21 / 25 / 29, 144 (B3 T383 H16) 33 / 38 / 50 -> 27 / 32 / 38.
+// From two workgroups per CU they overlap by themselves: N = 128 with 512
+// 78 / 87 / 118 -> 86 / 97 / 117. Exactly one per CU still gains (N = 64 with 256
+// 59 / 62 / 92 -> 41 / 50 / 65), but the line stays below it: a single sequence
+// that fills the card runs as it does inside a larger batch, bit for bit. Below 256
+// positions a group would get one tile or two (T 256: 9 / 12 / 14 -> 10 / 11 /
+// 11). N = 256 has no LDS for a second group.
+constexpr int kSplitGrid = 256;
+inline bool attn_split(int grid, int len, int N) { return grid < kSplitGrid && len >= 256 && N <= 128; }
 hipError_t launch_attn_fwd(const AttnFwdParams& p, int N, hipStream_t s);
 
 // Causal flash attention backward fused with the q/k RMSNorm + rotary
