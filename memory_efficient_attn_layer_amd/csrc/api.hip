@@ -46,7 +46,7 @@ Layout make_layout(const mea_desc& d, int pass) {
   L.wpk = take(4 * HN * C * 2);
   if (pass == MEA_PASS_FWD) {
     L.o = take(act);
-    L.qkn = take(2 * sizeof(float));
+    L.qkn = take(2 * mea::kNormSlots * sizeof(float));
   } else {
     L.dO = take(act);
     L.daq = take(act);
@@ -379,7 +379,7 @@ struct Prep {
 };
 hipError_t prepare(const mea_desc* d, const Varlen* var, const void* wq, const void* wk, const void* wv,
                    const void* wg, const void* wo, const float* f1, const float* f2, void* ws, const Layout& L,
-                   float* zero2, bf16_bits* wcatT, bf16_bits* woT, hipStream_t s, Prep* out) {
+                   float* norms, bf16_bits* wcatT, bf16_bits* woT, hipStream_t s, Prep* out) {
   mea::PrepParams p = {};
   p.wq = static_cast<const bf16_bits*>(wq);
   p.wk = static_cast<const bf16_bits*>(wk);
@@ -399,7 +399,7 @@ hipError_t prepare(const mea_desc* d, const Varlen* var, const void* wq, const v
     p.table_words = out->tab_rows * (int)(d->N / 4);
     out->tabp = p.tabp = at<bf16_bits>(ws, L.rot);
   }
-  p.zero2 = zero2;
+  p.norms = norms;
   if (var != nullptr) {
     p.cu = var->cu;
     p.nseq = var->nseq;

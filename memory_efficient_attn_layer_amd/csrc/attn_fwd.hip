@@ -114,7 +114,14 @@ __global__ __launch_bounds__(256 * SPLIT, SPLIT > 1 ? 1 : N <= 64 ? 4 : N == 128
 
   bool fixed = false;
   if (p.qk_norm2 != nullptr && p.sl2e == 1.0f) {
-    const float bound = sqrtf(p.qk_norm2[0] * p.qk_norm2[1]) * 1.01f;
+    uint32_t nq = 0, nk = 0;  // bit patterns, which order like the non-negative floats
+    const uint32_t* ns = reinterpret_cast<const uint32_t*>(p.qk_norm2);
+#pragma unroll
+    for (int i = 0; i < kNormSlots; ++i) {
+      nq = max(nq, ns[2 * i]);
+      nk = max(nk, ns[2 * i + 1]);
+    }
+    const float bound = sqrtf(__uint_as_float(nq) * __uint_as_float(nk)) * 1.01f;
     fixed = bound <= kFixedBound;
   }
 

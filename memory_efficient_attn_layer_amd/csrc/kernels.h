@@ -10,6 +10,16 @@ namespace mea {
 typedef uint16_t bf16_bits;
 
 // Input RMSNorm + q/k/v/g projection + q/k head RMSNorm + rotary + sigmoid.
+// The largest squared norms of the stored q and k rows, which bound every logit:
+// pairs of floats, workgroup w of the projection raising pair w % kNormSlots
+// by atomic max, and the attention taking the maximum over all of them. Atomics
+// on one address are served one after the other, about 12 ns each: with one
+// pair and an atomic per wave, 512 workgroups that end together waited 20 us for
+// them. Projection, us, one pair and four atomics a workgroup -> one pair and one
+// -> 16 pairs and one: M 8192 C 32 H 8 N 64 32.4 -> 15.8 -> 13.3, C 512 42.6 ->
+// 27.6 -> 26.4, M 4096 C 1024 H 16 54.7 -> 41.7 -> 41.9; 32 pairs, or pairs 256
+// bytes apart, measured like 16. They are two scalar loads in the attention.
+constexpr int kNormSlots = 16;
 struct ProjParams {
   const bf16_bits* x;                       // (M, C)
   // (H*N, C) weights: element (row, k) at row * w_row + (k / 32) * w_slab +
@@ -28,9 +38,7 @@ struct ProjParams {
   bf16_bits* sig;                           // (M, H*N)
   float* rx;                                // (M) or null
   float *rq, *rk;                           // (B, H, T) or null
-  // Largest squared norms of the stored q and k rows (2 floats, zeroed
-  // beforehand, raised with atomic max) or null.
-  float* qk_norm2;
+  float* qk_norm2;                          // norm slots (kNormSlots), zeroed beforehand, or null
   // Rotary row of every token (M), or null (row = t of the (B, T) layout):
   // packed sequences give each token its position inside its sequence.
   const int* tpos;
@@ -61,7 +69,7 @@ struct PrepParams {
   const float *f1, *f2;
   int table_words;
   bf16_bits* tabp;
-  float* zero2;                             // two floats to clear
+  float* norms;                             // norm slots to clear (kNormSlots), or null
   // tpos[m] = m - cu[s] for cu[s] <= m < cu[s+1] (packed sequences).
   const int* cu;
   int nseq, M;

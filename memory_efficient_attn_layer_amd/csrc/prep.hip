@@ -99,7 +99,8 @@ __host__ __device__ __forceinline__ PrepGrid prep_grid(const PrepParams& p) {
 
 __global__ __launch_bounds__(256) void prep_kernel(PrepParams p) {
   __shared__ bf16_bits tile[64][64 + 2];
-  if (p.zero2 != nullptr && blockIdx.x == 0 && threadIdx.x < 2) p.zero2[threadIdx.x] = 0.f;
+  if (p.norms != nullptr && blockIdx.x == 0)
+    for (int i = threadIdx.x; i < 2 * kNormSlots; i += 256) p.norms[i] = 0.f;
   const PrepGrid g = prep_grid(p);
   int blk = blockIdx.x;  // uniform: every block runs one job
   if (blk < g.wcat) {
@@ -143,7 +144,7 @@ hipError_t launch_prep(const PrepParams& p, hipStream_t s) {
   if (p.HN % 32 != 0 || p.C % 32 != 0) return hipErrorInvalidValue;
   const PrepGrid g = prep_grid(p);
   const int n = g.slab + g.tab + g.pos + g.wcat + g.wo;
-  if (n == 0 && p.zero2 == nullptr) return hipSuccess;
+  if (n == 0 && p.norms == nullptr) return hipSuccess;
   hipLaunchKernelGGL(prep_kernel, dim3(n > 0 ? n : 1), dim3(256), 0, s, p);
   return hipGetLastError();
 }

@@ -89,6 +89,7 @@ __global__ __launch_bounds__(256, 2) void qkvg_proj_kernel(ProjParams p) {
   constexpr int LOADS = (BF + BT) * BK / 8 / 64 / 4;  // load instructions per wave per slab
   __shared__ __attribute__((aligned(16))) bf16_bits smem[NS * STAGE];
   __shared__ float ssq_s[BT];
+  __shared__ float nrm_s[2][4];  // largest squared q and k row norms of the four waves
   __shared__ float xch[2][HALF ? 2 : 1][HALF ? BT : 1];  // [ss | norm][wf][token] (HALF)
 
   // Locals, not captures of the argument block: a lambda holding &p would
@@ -510,19 +511,24 @@ __global__ __launch_bounds__(256, 2) void qkvg_proj_kernel(ProjParams p) {
       epilogue(std::false_type{});
   }
   if (p.qk_norm2 != nullptr && ntl > 0) {
-    auto publish = [&](float v, int slot) {
+    // One atomic instruction per workgroup, on its slot (see kNormSlots).
+    auto row_max = [&](float v) {
       v = fmaxf(v, xor1(v));
       v = fmaxf(v, xor2(v));
       v = fmaxf(v, shfl_xor(v, 4));
-      v = fmaxf(v, shfl_xor(v, 8));
-      // Non-negative floats order like their bit patterns.
-      if (lane == 0) atomicMax(reinterpret_cast<unsigned int*>(p.qk_norm2) + slot, __float_as_uint(v));
+      return fmaxf(v, shfl_xor(v, 8));
     };
-    if (HALF) {
-      publish(nmax, 0);
-      publish(nmax_k, 1);
-    } else {
-      publish(nmax, wf);
+    const float nq = row_max(nmax), nk2 = HALF ? row_max(nmax_k) : 0.f;
+    if (lane == 0) {
+      nrm_s[HALF ? 0 : wf][wave] = nq;
+      nrm_s[HALF ? 1 : wf ^ 1][wave] = nk2;
+    }
+    __syncthreads();
+    if (tid < 2) {
+      const float v = fmaxf(fmaxf(nrm_s[tid][0], nrm_s[tid][1]), fmaxf(nrm_s[tid][2], nrm_s[tid][3]));
+      // Non-negative floats order like their bit patterns.
+      atomicMax(reinterpret_cast<unsigned int*>(p.qk_norm2) + 2 * (blockIdx.x % kNormSlots) + tid,
+                __float_as_uint(v));
     }
   }
 }
