@@ -249,11 +249,14 @@ __global__ __launch_bounds__(256, 2) void qkvg_proj_kernel(ProjParams p) {
       if (POS) return min(max(p.tpos[min(m, M - 1)], 0), p.t_max - 1);
       return tile_whole ? t0 + (m - m0) : (m < M ? m - (m / T) * T : 0);
     };
-    // N = 64: one slot of table rows, filled for block 0 at the start of the
+    // N <= 64: one slot of table rows, filled for block 0 at the start of the
     // epilogue and refilled, feature block by feature block, for block tb + 1
-    // as block tb consumes it. N = 128 (twice the rows) reads each feature
-    // block's rows just before use.
-    constexpr bool PREF = N == 64;
+    // as block tb (N = 32: the second of its two heads) consumes it. N = 128
+    // (twice the rows) reads each feature block's rows just before use: a slot
+    // for all of them spills 43 to 91 registers, for half of them 8 to 34, and
+    // ran 5 to 10% longer. N = 32 without the slot, us: M 2048 C 512 H 8 19.9,
+    // M 16384 H 16 51; with it 17.7, 46.
+    constexpr bool PREF = N <= 64;
     constexpr bool SLOT32 = PREF && !PK, SLOTW = PREF && PK;
     f32x4 tab1[SLOT32 ? GF : 1], tab2[SLOT32 ? GF : 1];
     u32x4 tabw[SLOTW ? GF : 1];
@@ -273,7 +276,7 @@ __global__ __launch_bounds__(256, 2) void qkvg_proj_kernel(ProjParams p) {
         tab2[SLOT32 ? j : 0] = tab_at(p.f2, tb, j);
       }
     };
-    // (f1, f2) of those features, from the slot (N = 64) or from memory.
+    // (f1, f2) of those features, from the slot (N <= 64) or from memory.
     auto tab_vals = [&](int tb, int j, f32x4& a1, f32x4& a2) {
       if (PK) {
         const u32x4 w = SLOTW ? tabw[SLOTW ? j : 0] : tabw_at(tb, j);
@@ -488,7 +491,7 @@ __global__ __launch_bounds__(256, 2) void qkvg_proj_kernel(ProjParams p) {
 #pragma unroll
         for (int gi = 0; gi < 4; ++gi) {
           if (gi < 2)
-            rot_block(tb, gi, -1);
+            rot_block(tb, gi, gi == 1 && tb + 1 < TB ? tb + 1 : -1);
           else
             plain_block(tb, gi);
           drain_pj(gi, tb);
