@@ -637,18 +637,16 @@ int bwd_impl(const mea_desc* d, const Varlen* var, const void* dy, const void* x
   dw.C = C;
   dw.HN = HN;
   dw.splits = mea::dw_splits(M, C, HN);
+  dw.dwq = static_cast<bf16_bits*>(dwq);
+  dw.dwk = static_cast<bf16_bits*>(dwk);
+  dw.dwv = static_cast<bf16_bits*>(dwv);
+  dw.dwg = static_cast<bf16_bits*>(dwg);
+  dw.dwo = static_cast<bf16_bits*>(dwo);
   MEA_TRY(timed(K_DW_PARTIAL, s, [&] { return mea::launch_dw_partial(dw, s); }));
-  mea::DwReduceParams dr;
-  dr.part = bf.part;
-  dr.dwq = static_cast<bf16_bits*>(dwq);
-  dr.dwk = static_cast<bf16_bits*>(dwk);
-  dr.dwv = static_cast<bf16_bits*>(dwv);
-  dr.dwg = static_cast<bf16_bits*>(dwg);
-  dr.dwo = static_cast<bf16_bits*>(dwo);
-  dr.C = C;
-  dr.HN = HN;
-  dr.splits = dw.splits;
-  MEA_TRY(timed(K_DW_REDUCE, s, [&] { return mea::launch_dw_reduce(dr, s); }));
+  if (dw.splits > 1) {
+    const mea::DwReduceParams dr = {bf.part, dw.dwq, dw.dwk, dw.dwv, dw.dwg, dw.dwo, C, HN, dw.splits};
+    MEA_TRY(timed(K_DW_REDUCE, s, [&] { return mea::launch_dw_reduce(dr, s); }));
+  }
 
   mea::DxParams dxp;
   dxp.da = da;

@@ -821,7 +821,10 @@ __device__ __forceinline__ bf16x8 dw_frag(const bf16_bits* slab, int f, int lane
 
 }  // namespace
 
-template <bool FAST>
+// DIRECT: one split, whose sums are the gradients: they leave as bf16 and no
+// reduction follows. C 2048 H 16 N 128, us: M 700 60.6 + 19.2 -> 59.2, M 4096
+// 243 + 21 -> 256.
+template <bool FAST, bool DIRECT>
 __global__ __launch_bounds__(512, 1) void dw_partial_kernel(DwParams p) {
   constexpr int STAGES = 3;
   __shared__ __attribute__((aligned(16))) bf16_bits smem[STAGES * 2 * kDwSlab];
@@ -948,6 +951,31 @@ __global__ __launch_bounds__(512, 1) void dw_partial_kernel(DwParams p) {
       for (int b = 0; b < 8; ++b) acc[a][b] = mfma(af[a], bfr[b], acc[a][b]);
   }
 
+  if constexpr (DIRECT) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      const int ib = i0 + wi * 64 + a * 16;  // 16 rows of one matrix (HN is a multiple of 32)
+      if (ib >= I) continue;
+      const int pj = prob1 ? 4 : ib / HN;
+      bf16_bits* dst = pj == 0 ? p.dwq : pj == 1 ? p.dwk : pj == 2 ? p.dwv : pj == 3 ? p.dwg : p.dwo;
+      dst += (size_t)(prob1 ? ib : ib - pj * HN) * J;
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        const int jb = j0 + wj * 128 + b * 16;
+        if (jb >= J) continue;
+        // Neighbouring lanes hold neighbouring columns: an even lane takes both
+        // of row 4g + r, an odd one both of row 4g + r + 1.
+        const int odd = c16 & 1;
+#pragma unroll
+        for (int r = 0; r < 4; r += 2) {
+          const float got = xor1(odd ? acc[a][b][r] : acc[a][b][r + 1]);
+          const uint32_t w = odd ? pack2(got, acc[a][b][r + 1]) : pack2(acc[a][b][r], got);
+          *reinterpret_cast<uint32_t*>(dst + (size_t)(4 * g + r + odd) * J + jb + (c16 & ~1)) = w;
+        }
+      }
+    }
+    return;
+  }
   const size_t per_split = (size_t)K4 * C + (size_t)C * HN;
   float* out = p.part + (size_t)z * per_split + (prob1 ? (size_t)K4 * C : 0);
 #pragma unroll
@@ -989,10 +1017,16 @@ hipError_t launch_dw_partial(const DwParams& p, hipStream_t s) {
   if (p.C % 32 != 0 || (4 * p.HN) % kDwTile != 0) return hipErrorInvalidValue;
   const int tiles = dw_tiles(p.C, p.HN);
   // The fast path reads dy's columns unclamped: whole tiles along C only.
-  if (p.da.T % kDwBK == 0 && p.HN % kDwTile == 0 && p.C % kDwTile == 0)
-    hipLaunchKernelGGL(dw_partial_kernel<true>, dim3(tiles * p.splits), dim3(512), 0, s, p);
+  const bool fast = p.da.T % kDwBK == 0 && p.HN % kDwTile == 0 && p.C % kDwTile == 0;
+  const dim3 grid(tiles * p.splits), block(512);
+  if (fast && p.splits == 1)
+    hipLaunchKernelGGL((dw_partial_kernel<true, true>), grid, block, 0, s, p);
+  else if (fast)
+    hipLaunchKernelGGL((dw_partial_kernel<true, false>), grid, block, 0, s, p);
+  else if (p.splits == 1)
+    hipLaunchKernelGGL((dw_partial_kernel<false, true>), grid, block, 0, s, p);
   else
-    hipLaunchKernelGGL(dw_partial_kernel<false>, dim3(tiles * p.splits), dim3(512), 0, s, p);
+    hipLaunchKernelGGL((dw_partial_kernel<false, false>), grid, block, 0, s, p);
   return hipGetLastError();
 }
 

@@ -243,14 +243,15 @@ struct DwParams {
   const bf16_bits* x;                       // (M, C)
   const bf16_bits* dy;                      // (M, C)
   const bf16_bits* z;                       // (M, HN)
-  float* part;                              // (splits, 4*HN*C + C*HN)
+  float* part;                              // (splits, 4*HN*C + C*HN) if splits > 1
+  bf16_bits *dwq, *dwk, *dwv, *dwg, *dwo;   // written if splits == 1
   int M, C, HN, splits;
 };
 // Token splits of the weight-gradient reduction for a shape (one workgroup
 // per CU over all output tiles); the workspace holds that many partials.
 int dw_splits(int M, int C, int HN);
 hipError_t launch_dw_partial(const DwParams& p, hipStream_t s);
-// Sums the partials and writes the five bf16 weight gradients.
+// Sums the partials (splits > 1) and writes the five bf16 weight gradients.
 struct DwReduceParams {
   const float* part;
   bf16_bits *dwq, *dwk, *dwv, *dwg, *dwo;
