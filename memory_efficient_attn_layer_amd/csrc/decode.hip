@@ -77,7 +77,8 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
   const int k_begin = blockIdx.y * per, k_end = min(k_begin + per, pos);
 
   // Rows of a block: a uniform base and the lane's offset; rows past the split
-  // read its last one (their scores are masked).
+  // read its last one. Their scores are masked, which leaves them a weight of 0,
+  // and their values are taken as 0 (an infinity times 0 is not).
   const bf16_bits* kc = p.k_cache + (size_t)bh * p.Tc * N;
   const bf16_bits* vc = p.v_cache + (size_t)bh * p.Tc * N;
   const uint32_t lane_off = j * N + 8 * c;
@@ -175,6 +176,11 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] *= alpha;
     m_run = m_new;
+    if (k0 + KB > k_end) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+        if (k0 + i * KPI + j >= k_end) vr[i] = u32x4{0u, 0u, 0u, 0u};
+    }
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const float pv = fast_exp2(sc[i] - m_new);  // 0 for keys past the split
