@@ -30,8 +30,10 @@
 // stretches before). Requesting a wave's first block before the epilogue needs
 // 152 registers, three waves per SIMD: no faster (75.2 us), and spilled to 128
 // 124 us.
-#include "kernels.h"
+#include <type_traits>
+
 #include "common.cuh"
+#include "kernels.h"
 
 namespace mea {
 
@@ -76,22 +78,8 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
   const int per = (pos + p.S * SPAN - 1) / (p.S * SPAN) * SPAN;
   const int k_begin = blockIdx.y * per, k_end = min(k_begin + per, pos);
 
-  // Rows of a block: a uniform base and the lane's offset; rows past the split
-  // read its last one. Their scores are masked, which leaves them a weight of 0,
-  // and their values are taken as 0 (an infinity times 0 is not).
   const bf16_bits* kc = p.k_cache + (size_t)bh * p.Tc * N;
   const bf16_bits* vc = p.v_cache + (size_t)bh * p.Tc * N;
-  const uint32_t lane_off = j * N + 8 * c;
-  auto load = [&](u32x4 (&r)[NI], const bf16_bits* src, int k0) {
-    if (k0 + KB <= k_end) {
-      const bf16_bits* base = src + (size_t)k0 * N;
-#pragma unroll
-      for (int i = 0; i < NI; ++i) r[i] = ld16(base + i * KPI * N + lane_off);
-    } else if (k0 < k_end) {
-#pragma unroll
-      for (int i = 0; i < NI; ++i) r[i] = ld16(src + (size_t)min(k0 + i * KPI + j, k_end - 1) * N + 8 * c);
-    }
-  };
 
   // Projection epilogue of this head, thread n < N owning feature n, the same
   // steps as the full-sequence kernel's: a = rx * (x W^T) with rx =
@@ -147,12 +135,25 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
   float m_run = -INFINITY, l_run = 0.f, o[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = 0.f;
-  for (int k0 = k_begin + wave * KB; k0 < k_end; k0 += SPAN) {
+  // One block of a wave, rows at a uniform base and the lane's offset. TAIL: its
+  // rows past the split are not read; their scores are masked and their values 0
+  // (a weight of 0 does not cancel an infinity).
+  const uint32_t lane_off = j * N + 8 * c;
+  auto block = [&](int k0, auto tail_tag) {
+    constexpr bool TAIL = decltype(tail_tag)::value;
     // The block's K and V rows are requested together (V does not depend on
     // the scores), so twice the bytes are in flight per wave.
     u32x4 kr[NI], vr[NI];
-    load(kr, kc, k0);
-    load(vr, vc, k0);
+    auto load = [&](u32x4 (&r)[NI], const bf16_bits* src) {
+      const bf16_bits* base = src + (size_t)k0 * N;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        if (TAIL) r[i] = u32x4{0u, 0u, 0u, 0u};
+        if (!TAIL || k0 + i * KPI + j < k_end) r[i] = ld16(base + i * KPI * N + lane_off);
+      }
+    };
+    load(kr, kc);
+    load(vr, vc);
     float sc[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) d = __builtin_fmaf(qv[e], kf[e], d);
       d = row_sum<KL>(d);
-      sc[i] = k0 + i * KPI + j < k_end ? d : -INFINITY;
+      sc[i] = !TAIL || k0 + i * KPI + j < k_end ? d : -INFINITY;
     }
     float mb = sc[0];
 #pragma unroll
@@ -176,11 +177,6 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] *= alpha;
     m_run = m_new;
-    if (k0 + KB > k_end) {
-#pragma unroll
-      for (int i = 0; i < NI; ++i)
-        if (k0 + i * KPI + j >= k_end) vr[i] = u32x4{0u, 0u, 0u, 0u};
-    }
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const float pv = fast_exp2(sc[i] - m_new);  // 0 for keys past the split
@@ -190,7 +186,10 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[e] = __builtin_fmaf(pv, vf[e], o[e]);
     }
-  }
+  };
+  int k0 = k_begin + wave * KB;
+  for (; k0 + KB <= k_end; k0 += SPAN) block(k0, std::false_type{});
+  if (k0 < k_end) block(k0, std::true_type{});
   // Sum over the key slots (lanes with the same chunk c). Every lane of a
   // slot holds the slot's l, so the sum over slots is the wave's l.
 #pragma unroll
