@@ -67,7 +67,7 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
   constexpr int NI = 8;           // load instructions per block
   constexpr int KB = NI * KPI;    // keys per block of one wave
   constexpr int SPAN = 4 * KB;    // keys per turn of the workgroup
-  __shared__ float qs[N], po[4][N], pm[4], pl[4], red[4][4];
+  __shared__ float qs[N], po[4][N], pm[4], pl[4], red[2][4];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane / KL, c = lane % KL;
@@ -85,13 +85,21 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
   // steps as the full-sequence kernel's: a = rx * (x W^T) with rx =
   // rsqrt(mean(x^2) + eps) (fast_triton_attn.py:29-32), per-head RMSNorm of q
   // and k (:102-106), rotary (:132-141) at row pos[b], q times qscale, v plain,
-  // sigmoid(g) (:123).
+  // sigmoid(g) (:123). The squares of q and k are taken after rx, as there is no
+  // bound on those of the products themselves; a wave sums them over the whole
+  // head (NL features a lane), without another barrier.
   const int n = tid < N ? tid : 0;
-  const float live = tid < N ? 1.f : 0.f;
-  const float* a = p.a + (size_t)b * 4 * HN + h * N + n;
-  const float aq = a[0] * live;
-  const float ak = first ? a[HN] * live : 0.f;
+  constexpr int NL = N > 64 ? N / 64 : 1;
+  const float* ah = p.a + (size_t)b * 4 * HN + h * N;
+  const float* a = ah + n;
+  const float aq = tid < N ? a[0] : 0.f, ak = first && tid < N ? a[HN] : 0.f;
   const float av = first ? a[2 * HN] : 0.f, ag = first ? a[3 * HN] : 0.f;
+  float aql[NL], akl[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    aql[i] = NL == 1 ? aq : ah[64 * i + lane];
+    akl[i] = NL == 1 ? ak : first ? ah[HN + 64 * i + lane] : 0.f;
+  }
   const int row = min(pos, p.t_max - 1);
   const float f1 = p.f1[(size_t)row * N + n], f2 = p.f2[(size_t)row * N + n];
   float ss = 0.f;
@@ -101,17 +109,21 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss = __builtin_fmaf(xv[e], xv[e], ss);
   }
-  const float s0 = wave_sum(ss), s1 = wave_sum(aq * aq), s2 = wave_sum(ak * ak);
-  if (lane == 0) {
-    red[0][wave] = s0;
-    red[1][wave] = s1;
-    red[2][wave] = s2;
-  }
+  ss = wave_sum(ss);
+  if (lane == 0) red[0][wave] = ss;
   __syncthreads();
   auto total = [&](int i) { return (red[i][0] + red[i][1]) + (red[i][2] + red[i][3]); };
   const float rx = rsqrtf(total(0) / (float)p.C + p.eps);
-  const float qh = aq * rx * rsqrtf(rx * rx * total(1) * p.inv_n + p.eps);
-  const float kh = ak * rx * rsqrtf(rx * rx * total(2) * p.inv_n + p.eps);
+  float sq = 0.f, sk = 0.f;
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const float q = aql[i] * rx, k = akl[i] * rx;
+    sq = __builtin_fmaf(q, q, sq);
+    sk = __builtin_fmaf(k, k, sk);
+  }
+  sq = wave_sum(sq);
+  if (first) sk = wave_sum(sk);
+  const float qh = aq * rx * rsqrtf(sq * p.inv_n + p.eps), kh = ak * rx * rsqrtf(sk * p.inv_n + p.eps);
   const bf16_bits qb = f2bf((qh * f1 + xor1(qh) * f2) * p.qscale);
   float score = 0.f, vnew = 0.f;  // this feature's share of q . k_new; v_new
   if (first) {
@@ -205,7 +217,7 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
   if (lane == 0) {
     pm[wave] = m_run;
     pl[wave] = l_run;
-    red[3][wave] = score;
+    red[1][wave] = score;
   }
   __syncthreads();
   if (tid >= N) return;
@@ -223,7 +235,7 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
   if (first) {
     float* own = p.part + ((size_t)bh * (p.S + 1) + p.S) * (N + 4);
     own[n] = vnew;
-    if (n == 0) *reinterpret_cast<f32x4*>(own + N) = f32x4{total(3), 1.f, 0.f, 0.f};
+    if (n == 0) *reinterpret_cast<f32x4*>(own + N) = f32x4{total(1), 1.f, 0.f, 0.f};
   }
 }
 
