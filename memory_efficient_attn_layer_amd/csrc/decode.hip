@@ -184,14 +184,14 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
     for (int off = KL; off < 64; off <<= 1) mb = fmaxf(mb, shfl_xor(mb, off));
     // The block's first key is valid, so mb is finite.
     const float m_new = fmaxf(m_run, mb);
-    const float alpha = fast_exp2(m_run - m_new);  // 0 on the first block
+    const float alpha = exp2f(m_run - m_new);  // 0 on the first block
     l_run *= alpha;
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] *= alpha;
     m_run = m_new;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const float pv = fast_exp2(sc[i] - m_new);  // 0 for keys past the split
+      const float pv = exp2f(sc[i] - m_new);  // 0 for keys past the split
       l_run += pv;
       float vf[8];
       unpack8(vr[i], vf);
@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
   float num = 0.f, den = 0.f;
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
-    const float wt = pm[w] == -INFINITY ? 0.f : fast_exp2(pm[w] - M);  // a wave without keys
+    const float wt = pm[w] == -INFINITY ? 0.f : exp2f(pm[w] - M);  // a wave without keys
     num = __builtin_fmaf(wt, po[w][n], num);
     den = __builtin_fmaf(wt, pl[w], den);
   }
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(256) void attn_decode_combine_kernel(DecodeParams p
 #pragma unroll 4
   for (int s = gi; s < parts; s += G) {
     const float* ps = part + (size_t)s * (N + 4);
-    const float w = fast_exp2(ps[N] - M);
+    const float w = exp2f(ps[N] - M);
     num = __builtin_fmaf(w, ps[n], num);
     den = __builtin_fmaf(w, ps[N + 1], den);
   }

@@ -1,5 +1,6 @@
 """The decode step on values at the ends of their range: infinities in the
-cache, products whose squares leave fp32."""
+cache, products whose squares leave fp32, softmax weights below the normal
+numbers."""
 import pytest
 import torch
 
@@ -54,3 +55,29 @@ def test_products_whose_squares_leave_fp32(N, xs, wsc, eps):
     y = decode_step((x * xs).cuda(), *(w.cuda() for w in ws), f1.cuda(), f2.cuda(), H, N, pos, KVCache(kc, vc), eps)
     assert_out_close("k row", kc.cpu()[at, :, pos], kn)
     assert_out_close("y", y, ref)
+
+
+@pytest.mark.parametrize("N", [32, 64, 128, 256])
+@pytest.mark.parametrize("pos", [1, 2], ids=["across-splits", "within-a-wave"])
+def test_weights_below_the_normal_numbers_count(N, pos):
+    """A key about 2^-135 behind the best one, with values of 2^127. Rounding q
+    to bf16 moves its exponent by at most 2^-9 of 135 plus the new key's share,
+    under half a unit: a factor of 1.5."""
+    ws, f1, f2, x, k, v = _inputs(N)
+    ws[2] = torch.zeros_like(ws[2])
+    xn = ob.rms_norm(x.double(), 1e-6)
+    q, kn, g = (((xn @ ws[i].double().t()).reshape(1, 1, H, N)) for i in (0, 1, 3))
+    q, kn = (ob.rotary(ob.rms_norm(t, 1e-6), f1[pos:pos + 1].double(), f2[pos:pos + 1].double())[0, 0] for t in (q, kn))
+    unit = 1.4426950408889634 / N ** 0.5  # log2 units of a logit
+    far = (q * kn.bfloat16().double()).sum(-1, keepdim=True).mul(unit).clamp(min=0.0) - 135.0
+    k[0, :, 0] = (q * far / (unit * q.square().sum(-1, keepdim=True))).bfloat16()
+    k[0, :, 1:pos] = 0.0  # a logit of 0
+    v[0] = 0.0
+    v[0, :, 0] = 2.0 ** 127
+    keys = torch.cat((k[0, :, :pos].double(), kn[:, None]), dim=1)
+    p = torch.softmax((keys @ q[:, :, None])[..., 0] / N ** 0.5, dim=-1)
+    ref = ((p[:, :1] * 2.0 ** 127) * torch.sigmoid(g[0, 0])).reshape(1, H * N) @ ws[4].double().t()
+    assert 2.0 ** -136 < float(p[:, 0].min()) and float(p[:, 0].max()) < 2.0 ** -128
+    y = _decode(x, ws, f1, f2, [pos], k, v, N).double()
+    ratio = float((y * ref).sum() / ref.square().sum())
+    assert 1 / 1.5 < ratio < 1.5
