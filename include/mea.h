@@ -243,7 +243,9 @@ size_t mea_decode_workspace_bytes(const mea_desc* d);
  *   x                 (B, C) bf16            the new tokens
  *   wq .. wo, f1, f2  as in mea_fwd
  *   pos               (B) int32, device      0 <= pos[b] < Tc; values outside
- *                                            are clamped to that range
+ *                                            are clamped to that range for
+ *                                            the cache, to 0 .. T_max - 1 for
+ *                                            the rotary row
  *   k_cache, v_cache  (B, H, Tc, N) bf16     rows 0..pos[b]-1 hold the
  *                                            earlier tokens (mea_prefill or
  *                                            earlier steps); row pos[b] is

@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
     aql[i] = NL == 1 ? aq : ah[64 * i + lane];
     akl[i] = NL == 1 ? ak : first ? ah[HN + 64 * i + lane] : 0.f;
   }
-  const int row = min(pos, p.t_max - 1);
+  const int row = min(max(p.pos[b], 0), p.t_max - 1);
   const float f1 = p.f1[(size_t)row * N + n], f2 = p.f2[(size_t)row * N + n];
   float ss = 0.f;
   for (int i = tid * 8; i < p.C; i += 2048) {

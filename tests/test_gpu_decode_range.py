@@ -1,9 +1,12 @@
 """The decode step on values at the ends of their range: infinities in the
 cache, products whose squares leave fp32, softmax weights below the normal
-numbers."""
+numbers, positions past the capacity."""
+import ctypes
+
 import pytest
 import torch
 
+from memory_efficient_attn_layer_amd import _lib
 from memory_efficient_attn_layer_amd.decode import KVCache, decode_step
 from memory_efficient_attn_layer_amd.yarn import rotary_tables
 from oracle import block as ob
@@ -81,3 +84,28 @@ def test_weights_below_the_normal_numbers_count(N, pos):
     y = _decode(x, ws, f1, f2, [pos], k, v, N).double()
     ratio = float((y * ref).sum() / ref.square().sum())
     assert 1 / 1.5 < ratio < 1.5
+
+
+def test_position_past_the_capacity():
+    """Clamped to the capacity for the cache, to the tables for the rotary row."""
+    N, cap, pos = 64, 40, 45
+    ws, f1, f2, x, k, v = _inputs(N)
+    k, v = k[:, :, :cap].contiguous(), v[:, :, :cap].contiguous()
+    lib, dev = _lib.load(), [t.cuda() for t in (x, *ws, f1, f2)]
+
+    def run(t_max, f1, f2, p):
+        d = _lib.desc(1, cap, C, H, N, t_max, 1e-6)
+        need = lib.mea_decode_workspace_bytes(ctypes.byref(d))
+        kc, vc, y = k.cuda(), v.cuda(), torch.empty(1, C, dtype=torch.bfloat16, device="cuda")
+        scratch = torch.empty(need, dtype=torch.uint8, device="cuda")
+        at = torch.tensor([p], dtype=torch.int32, device="cuda")
+        rc = lib.mea_decode(ctypes.byref(d), *(t.data_ptr() for t in dev[:6]), f1.data_ptr(), f2.data_ptr(), at.data_ptr(),
+                            kc.data_ptr(), vc.data_ptr(), y.data_ptr(), scratch.data_ptr(), need, _lib.stream_of(y.device))
+        assert rc == 0, _lib.strerror(rc)
+        return y.cpu(), kc.cpu(), vc.cpu()
+
+    moved = [t[:cap].clone() for t in dev[6:]]
+    for t, full in zip(moved, dev[6:]):
+        t[cap - 1] = full[pos]
+    for got, want in zip(run(CAP, dev[6], dev[7], pos), run(cap, *moved, cap - 1)):
+        assert torch.equal(got, want)
