@@ -6,7 +6,7 @@ import torch
 
 from memory_efficient_attn_layer_amd import stages
 from memory_efficient_attn_layer_amd.synthetic import Workload
-from tests.parity_util import assert_out_close, check_block
+from tests.parity_util import assert_grad_close, assert_out_close, check_block
 from tests.test_gpu_varlen import _gpu_varlen, _inputs, _oracle
 
 pytestmark = pytest.mark.gpu
@@ -40,3 +40,18 @@ def test_packed_sequences_of_uneven_lengths():
     got, ref = _gpu_varlen(inp, lens, H, N, table_grad=False), _oracle(inp, lens, H, N)
     for n in ("y", "dx", "dwq", "dwk", "dwv", "dwg", "dwo"):
         assert_out_close(n, got[n], ref[n], tol=3e-2)
+
+
+def test_packed_table_gradients():
+    lens, C, H, N = [300, 1, 0, 257, 90], 64, 2, 64
+    inp = _inputs(lens, C, H, N, t_max=310, seed=5)
+    got, ref = _gpu_varlen(inp, lens, H, N), _oracle(inp, lens, H, N)
+    for n in ("df1", "df2"):
+        assert_grad_close(n, got[n][:300], ref[n][:300])
+        assert not bool(got[n][300:].any())
+
+
+@pytest.mark.parametrize("B,T,H,N", [(17, 300, 5, 64), (16, 256, 8, 64), (17, 383, 5, 128), (8, 512, 8, 128)],
+                         ids=["n64-255", "n64-256", "n128-255", "n128-256"])
+def test_both_sides_of_the_grid_line(B, T, H, N):
+    check_block(Workload(99, "line", B, T, 64, H, N), seed=T, table_grad=False)
