@@ -19,7 +19,7 @@ inline size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
 // Byte offsets of every transient inside the workspace.
 struct Layout {
-  size_t q, k, v, sig, tpos, o, qkn;         // forward (tpos: packed sequences only)
+  size_t q, k, v, sig, tpos, qkn;            // forward (tpos: packed sequences only)
   size_t rot;                                // packed bf16 tables (tables_bf16 only)
   size_t wpk;                                // k-slab-major copies of Wq, Wk, Wv, Wg
   size_t dO, daq, dag;                       // backward (da_k, da_v overwrite k, v)
@@ -45,7 +45,6 @@ Layout make_layout(const mea_desc& d, int pass) {
   if (d.tables_bf16 != 0) L.rot = take((size_t)d.T * (size_t)d.N * 4);
   L.wpk = take(4 * HN * C * 2);
   if (pass == MEA_PASS_FWD) {
-    L.o = take(act);
     L.qkn = take(2 * mea::kNormSlots * sizeof(float));
   } else {
     L.dO = take(act);
@@ -60,7 +59,8 @@ Layout make_layout(const mea_desc& d, int pass) {
     L.delta = take(stat);
     L.woT = take(HN * C * 2);
     L.wcatT = take(C * 4 * HN * 2);
-    L.part = take((size_t)mea::dw_splits((int)M, (int)C, (int)HN) * (4 * HN * C + C * HN) * 4);
+    const int splits = mea::dw_splits((int)M, (int)C, (int)HN);  // one split leaves no partials
+    L.part = take(splits > 1 ? (size_t)splits * (4 * HN * C + C * HN) * 4 : 0);
     if (mea::dx_tile_tokens((int)M, (int)C, (int)HN) != 0) {
       // The tiled dx leaves fp32 rows and dot products for its second pass,
       // over the dW partials (dead by then) and as far past them as needed.

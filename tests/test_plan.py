@@ -16,3 +16,18 @@ def test_plan_matches_the_library(which, B, T, T_max, T_ws):
         assert n == lib.mea_workspace_bytes(ctypes.byref(_lib.desc(B, T, 96, 2, 64, T_ws, 1e-6, 0, b16)), which)
     d, n = _lib.decode_plan(max(B, 1), T, 96, 2, 64, 1e-6, 0)
     assert n == lib.mea_decode_workspace_bytes(ctypes.byref(d)) > 0
+
+
+def test_workspaces_hold_what_the_kernels_touch():
+    """No rows for an O that only a caller's o_save takes; no fp32 weight
+    gradients where one token split writes them as bf16."""
+    lib = _lib.load()
+    d = _lib.desc(4, 4096, 1024, 16, 64, 4096, 1e-6)
+    act, weights = 4 * 4096 * 1024 * 2, 4 * 1024 * 1024 * 2
+    fwd = lib.mea_workspace_bytes(ctypes.byref(d), _lib.MEA_PASS_FWD)
+    assert 4 * act + weights < fwd < 4 * act + weights + act // 2  # q, k, v, sig and the packed weights
+    B, T, C, HN = 1, 256, 2048, 2048
+    d = _lib.desc(B, T, C, 16, 128, T, 1e-6)
+    bwd = lib.mea_workspace_bytes(ctypes.byref(d), _lib.MEA_PASS_BWD)
+    known = 7 * T * HN * 2 + (4 + 4 + 1) * HN * C * 2 + T * C * 4  # rows, three weight layouts, the tiled dx's sums
+    assert known < bwd < known + HN * C * 4
