@@ -168,12 +168,12 @@ T* at(void* ws, size_t off) {
 enum KernelId {
   K_QKVG_PROJ, K_ATTN_FWD, K_GATE_OPROJ, K_PREP, K_DZ_GATE_BWD,
   K_ATTN_BWD_DQ, K_ATTN_BWD_DKDV, K_DW_PARTIAL, K_DW_REDUCE, K_DX,
-  K_ATTN_DECODE, K_DECODE_COMBINE, K_SKINNY_GEMM, K_TABLE_GRAD, K_COUNT
+  K_ATTN_DECODE, K_DECODE_COMBINE, K_SKINNY_GEMM, K_TABLE_GRAD, K_TABLE_ROWS, K_COUNT
 };
 const char* const kKernelNames[K_COUNT] = {
     "qkvg_proj", "attn_fwd", "gate_oproj", "prep", "dz_gate_bwd",
     "attn_bwd_dq", "attn_bwd_dkdv", "dw_partial", "dw_reduce", "dx",
-    "attn_decode", "attn_decode_combine", "skinny_gemm", "table_grad"};
+    "attn_decode", "attn_decode_combine", "skinny_gemm", "table_grad", "table_rows"};
 
 struct ProfRec {
   int kernel;
@@ -732,8 +732,11 @@ int mea_table_rows(const void* f1, const void* f2, int64_t rows, int64_t N, floa
   const int rc = check_ptrs({f1, f2, f1_out, f2_out});
   if (rc != MEA_OK) return rc;
   if (rows < 1 || N < 8 || N % 8 != 0 || rows > (INT64_C(1) << 31) / N - 1) return MEA_ERR_SHAPE;
-  MEA_TRY(mea::launch_table_rows(static_cast<const bf16_bits*>(f1), static_cast<const bf16_bits*>(f2), (int)(rows * N),
-                                 f1_out, f2_out, static_cast<hipStream_t>(stream)));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  MEA_TRY(timed(K_TABLE_ROWS, s, [&] {
+    return mea::launch_table_rows(static_cast<const bf16_bits*>(f1), static_cast<const bf16_bits*>(f2), (int)(rows * N),
+                                  f1_out, f2_out, s);
+  }));
   return MEA_OK;
 }
 

@@ -3,6 +3,7 @@ their tiles, and against the row-owning forms that larger calls take."""
 import pytest
 import torch
 
+from memory_efficient_attn_layer_amd import _lib
 from memory_efficient_attn_layer_amd.attention import _tables32
 from memory_efficient_attn_layer_amd.decode import KVCache, prefill
 from memory_efficient_attn_layer_amd.synthetic import Workload, make_inputs
@@ -58,6 +59,14 @@ def test_table_rows_are_the_fp32_values(T, N, rows):
     wide = torch.randn(T, 2 * N, device="cuda", generator=g).bfloat16()
     o1, o2 = _tables32(wide[:, :N], wide[:, N:], rows)
     assert torch.equal(o1, wide[:rows, :N].float()) and torch.equal(o2, wide[:rows, N:].float())
+
+
+def test_the_profile_counts_the_table_launch():
+    f = torch.ones(40, 64, device="cuda", dtype=torch.bfloat16)
+    _lib.profile_enable(True)
+    _tables32(f, f, 40)
+    _lib.profile_enable(False)
+    assert {k: n for k, (n, _) in _lib.profile_read().items()} == {"table_rows": 1}
 
 
 @pytest.mark.parametrize("H,N", [(2, 32), (3, 64), (2, 128), (1, 256)], ids=lambda v: str(v))
