@@ -417,29 +417,29 @@ __global__ __launch_bounds__(256 * SPLIT, SPLIT > 1 ? 1 : N <= 64 ? 3 : N == 256
       }
       if (j - grp < nkv) __syncthreads();  // every group passes the same barriers
     } else {
-    issue_tile(0, 0);
-    wait_vmcnt0();  // also retires the q/dO fragment loads
-    __syncthreads();
-    int j = 0;
-    for (; j < nfull; ++j) {
-      if (j + 1 < nkv) issue_tile((j + 1) * BKV, (j + 1) & 1);
-      const bf16_bits* ks_t = smem + (j & 1) * 2 * TILE;
-      step(ks_t, ks_t + TILE, 0, j * BKV, std::false_type{});
-      step(ks_t, ks_t + TILE, 1, j * BKV + 32, std::false_type{});
-      wait_vmcnt0();
+      issue_tile(0, 0);
+      wait_vmcnt0();  // also retires the q/dO fragment loads
       __syncthreads();
-    }
-    for (; j < nkv; ++j) {
-      if (j + 1 < nkv) issue_tile((j + 1) * BKV, (j + 1) & 1);
-      const bf16_bits* ks_t = smem + (j & 1) * 2 * TILE;
-#pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        const int kb0 = j * BKV + st * 32;
-        if (kb0 <= q0w + QW - 1) step(ks_t, ks_t + TILE, st, kb0, std::true_type{});
+      int j = 0;
+      for (; j < nfull; ++j) {
+        if (j + 1 < nkv) issue_tile((j + 1) * BKV, (j + 1) & 1);
+        const bf16_bits* ks_t = smem + (j & 1) * 2 * TILE;
+        step(ks_t, ks_t + TILE, 0, j * BKV, std::false_type{});
+        step(ks_t, ks_t + TILE, 1, j * BKV + 32, std::false_type{});
+        wait_vmcnt0();
+        __syncthreads();
       }
-      wait_vmcnt0();
-      __syncthreads();
-    }
+      for (; j < nkv; ++j) {
+        if (j + 1 < nkv) issue_tile((j + 1) * BKV, (j + 1) & 1);
+        const bf16_bits* ks_t = smem + (j & 1) * 2 * TILE;
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+          const int kb0 = j * BKV + st * 32;
+          if (kb0 <= q0w + QW - 1) step(ks_t, ks_t + TILE, st, kb0, std::true_type{});
+        }
+        wait_vmcnt0();
+        __syncthreads();
+      }
     }
 
     // Stage dQ (times the softmax scale) as fp32 rows, then the q chain. With
@@ -777,10 +777,10 @@ __global__ __launch_bounds__(256 * SPLIT, SPLIT > 1 ? 1 : N <= 64 ? 3 : N == 128
       for (; it < nq; it += SPLIT) tile(it, std::true_type{});
       if (it - grp < nq) __syncthreads();  // every group passes the same barriers
     } else {
-    int it = 0;
-    if (nfull > 0 && (T - k0) % BQ != 0) tile(it++, std::true_type{});
-    for (; it < nfull; ++it) tile(it, std::false_type{});
-    for (; it < nq; ++it) tile(it, std::true_type{});
+      int it = 0;
+      if (nfull > 0 && (T - k0) % BQ != 0) tile(it++, std::true_type{});
+      for (; it < nfull; ++it) tile(it, std::false_type{});
+      for (; it < nq; ++it) tile(it, std::true_type{});
     }
 
     // Epilogue per 32-key block: stage dV (then dK * scale) as fp32 rows and run

@@ -392,12 +392,12 @@ __global__ __launch_bounds__(256 * SPLIT, SPLIT > 1 ? 1 : N <= 64 ? 4 : N == 128
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4)
           sx[(db * 4 + r4) * 64] = f32x4{o[0][db][4 * r4], o[0][db][4 * r4 + 1], o[0][db][4 * r4 + 2], o[0][db][4 * r4 + 3]};
-      sx_ml[0][SPLIT > 1 ? me : 0] = m_i[0];
-      sx_ml[SPLIT > 1 ? 1 : 0][SPLIT > 1 ? me : 0] = l_i[0];
+      sx_ml[0][me] = m_i[0];
+      sx_ml[1][me] = l_i[0];
     }
     __syncthreads();
     if (grp == 0) {
-      const float m1 = sx_ml[0][SPLIT > 1 ? me : 0], l1 = sx_ml[SPLIT > 1 ? 1 : 0][SPLIT > 1 ? me : 0];
+      const float m1 = sx_ml[0][me], l1 = sx_ml[1][me];
       const float m = fmaxf(m_i[0], m1), a0 = fast_exp2(m_i[0] - m), a1 = fast_exp2(m1 - m);
       m_i[0] = m;
       l_i[0] = l_i[0] * a0 + l1 * a1;
