@@ -59,8 +59,9 @@ def kernel_work(w):
     pair = 2.0 * B * H * N * T * (T + 1) / 2  # flops of one causal (T x T x N) product
     return {
         "qkvg_proj": dict(flops=2.0 * M * C * 4 * HN, bytes=2.0 * M * C + 2.0 * 4 * M * HN),
-        "attn_fwd": dict(flops=2 * pair, bytes=2.0 * 4 * M * HN),
-        "gate_oproj": dict(flops=2.0 * M * HN * C, bytes=2.0 * 2 * M * HN + 2.0 * M * C),
+        # reads q, k, v, sigmoid(a_g); writes z = O * sigmoid(a_g) and, for a backward, O
+        "attn_fwd": dict(flops=2 * pair, bytes=2.0 * (6 if w.backward else 5) * M * HN),
+        "gate_oproj": dict(flops=2.0 * M * HN * C, bytes=2.0 * M * HN + 2.0 * M * C),
         # reads dy, O, sigmoid(a_g); writes dO, da_g and z = O * sigmoid(a_g)
         "dz_gate_bwd": dict(flops=2.0 * M * C * HN, bytes=2.0 * M * C + 2.0 * 5 * M * HN),
         "attn_bwd_dq": dict(flops=1 * pair, bytes=2.0 * 5 * M * HN),

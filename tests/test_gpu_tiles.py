@@ -3,8 +3,8 @@ their tiles, and against the row-owning forms that larger calls take."""
 import pytest
 import torch
 
-from memory_efficient_attn_layer_amd import _lib
-from memory_efficient_attn_layer_amd.attention import _tables32
+from memory_efficient_attn_layer_amd import _lib, stages
+from memory_efficient_attn_layer_amd.attention import FusedAttentionFunction, _tables32
 from memory_efficient_attn_layer_amd.decode import KVCache, prefill
 from memory_efficient_attn_layer_amd.synthetic import Workload, make_inputs
 from tests.parity_util import check_block, gpu_block
@@ -37,6 +37,19 @@ def test_tiled_and_row_owning_forms_return_the_same_bits(B, C, H, N):
         one = dict(inp, x=inp["x"][b:b + 1], dy=inp["dy"][b:b + 1])
         got = gpu_block(one, H, N, table_grad=False)
         assert torch.equal(got["y"], full["y"][b:b + 1]) and torch.equal(got["dx"], full["dx"][b:b + 1])
+
+
+@pytest.mark.parametrize("B,T,C,H,N", [(2, 130, 96, 4, 64), (3, 300, 1056, 2, 128), (260, 128, 256, 2, 64), (130, 128, 768, 4, 32)],
+                         ids=["tiled", "tiled-wide", "rows-256", "rows-768"])
+def test_output_projection_of_the_block_is_the_stage(B, T, C, H, N):
+    """The block's ungated output projection (tiled, row-owning) on z = O * sig from
+    the attention's epilogue against the stand-alone gated stage on O and sig."""
+    inp = {n: t.cuda() for n, t in make_inputs(Workload(99, "stage", B, T, C, H, N), seed=C).items()}
+    w = [inp[n] for n in ("wq", "wk", "wv", "wg", "wo")]
+    y = FusedAttentionFunction.apply(inp["x"].requires_grad_(True), *w, inp["f1"], inp["f2"], H, N)
+    o = y.grad_fn.saved_tensors[-2]
+    sig = stages.qkvg_proj(inp["x"].detach(), *w[:4], inp["f1"].float(), inp["f2"].float(), H, N)[3]
+    assert torch.equal(stages.gate_oproj(o, sig, w[4], H, N), y)
 
 
 def test_projection_from_packed_and_row_major_weights_is_the_same():
