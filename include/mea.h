@@ -211,9 +211,9 @@ int mea_table_rows(const void* f1, const void* f2, int64_t rows, int64_t N,
 
 /*
  * Prefill of a KV cache: the inference forward of a whole prompt (mea_fwd
- * with o_save = lse_save = NULL, same workspace) that also copies the
- * prompt's k and v rows, exactly as the attention consumed them, into rows
- * 0..T-1 of the caller's caches. No counterpart in the reference, which
+ * with o_save = lse_save = NULL, same workspace) that writes the prompt's k
+ * and v rows, exactly as the attention then reads them, to rows 0..T-1 of the
+ * caller's caches. No counterpart in the reference, which
  * trains only; it is the prompt half of the decode step below.
  *
  *   x .. f2, y           as in mea_fwd (d->T = prompt length)
@@ -260,8 +260,8 @@ int mea_decode(const mea_desc* d, const void* x, const void* wq,
 
 /*
  * mea_decode without a workspace argument: the step's scratch (the new
- * tokens' projections, q/k/v/gate rows and the split-attention partials,
- * mea_decode_workspace_bytes(d) bytes) lives in a static device buffer of
+ * tokens' projections, gate and gated output rows and the split-attention
+ * partials, mea_decode_workspace_bytes(d) bytes) lives in a static device buffer of
  * MEA_STATIC_SCRATCH_BYTES inside the library, so a call allocates nothing
  * and needs no caller-provided scratch. No counterpart in the reference; it
  * is for callers that cannot allocate device memory: serving loops with a
@@ -312,7 +312,10 @@ int mea_attn_fwd(const mea_desc* d, const void* q, const void* k,
 
 /*
  * Stage: output gate and projection, y = (o * sig) W_o^T. Replaces
- * gate_repack_kernel (fast_triton_attn.py:146-176) and F.linear (:460).
+ * gate_repack_kernel (fast_triton_attn.py:146-176) and F.linear (:460). The
+ * block forms o * sig in the attention's epilogue and runs ungated forms of
+ * this product; the stage has a kernel of its own that forms it on the way in,
+ * with the same rounding.
  *
  *   o, sig   (B, T, H*N) bf16
  *   wo       (C, H*N) bf16

@@ -37,8 +37,8 @@ HIPCC_FLAGS = [
     f"-I{INCLUDE}",
 ]
 
-# Per-source flags. tilegemm: its kernels run one wave per SIMD, where the
-# compiler would keep the MFMA accumulators in AGPRs and move them between
+# Per-source flags. tilegemm: its kernels run one or two waves per SIMD, where
+# the compiler would keep the MFMA accumulators in AGPRs and move them between
 # register files in the main loop (232 moves; none with VGPR accumulators).
 SOURCE_FLAGS = {"tilegemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 

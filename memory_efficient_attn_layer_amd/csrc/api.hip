@@ -762,8 +762,9 @@ namespace {
 
 // Decode workspace: the raw products [a_q|a_k|a_v|a_g] (B x 4HN fp32), the
 // new token's sigmoid(g) and gated attention output (B x H*N bf16 each) and the
-// split partials, with room for one more bf16 row and for more splits than
-// decode_splits makes (callers and the static scratch size by this formula).
+// split partials. The total is also what mea_decode_static compares with its
+// buffer: it counts one bf16 row and more splits than the kernels use, so that
+// the shapes that entry point takes do not change with the split rule.
 struct DecLayout {
   size_t a, sig, z, part, total;
 };

@@ -9,7 +9,6 @@ namespace mea {
 
 typedef uint16_t bf16_bits;
 
-// Input RMSNorm + q/k/v/g projection + q/k head RMSNorm + rotary + sigmoid.
 // The largest squared norms of the stored q and k rows, which bound every logit:
 // pairs of floats, workgroup w of the projection raising pair w % kNormSlots
 // by atomic max, and the attention taking the maximum over all of them. Atomics
@@ -20,6 +19,8 @@ typedef uint16_t bf16_bits;
 // 27.6 -> 26.4, M 4096 C 1024 H 16 54.7 -> 41.7 -> 41.9; 32 pairs, or pairs 256
 // bytes apart, measured like 16. They are two scalar loads in the attention.
 constexpr int kNormSlots = 16;
+
+// Input RMSNorm + q/k/v/g projection + q/k head RMSNorm + rotary + sigmoid.
 struct ProjParams {
   const bf16_bits* x;                       // (M, C)
   // (H*N, C) weights: element (row, k) at row * w_row + (k / 32) * w_slab +
@@ -104,15 +105,23 @@ constexpr float kFixedBound = 60.0f;
 // Whether the attention kernels run two wave groups per workgroup (SPLIT). A
 // grid below one workgroup per CU is bound by the serial chain of its longest
 // workgroup (load, QK, softmax, PV per tile), so halving that chain pays.
-// Forward / dQ / dK,dV, one group -> two (us): N = 64 with 128 workgroups
-// (T 1024) 33 / 33 / 48 -> 24 / 28 / 35; N = 128 with 96 (B1 T768 H16)
-// 25 / 28 / 38 -> 21 / 25 / 29, 144 (B3 T383 H16) 33 / 38 / 50 -> 27 / 32 / 38.
-// From two workgroups per CU they overlap by themselves: N = 128 with 512
-// 78 / 87 / 118 -> 86 / 97 / 117. Exactly one per CU still gains (N = 64 with 256
-// 59 / 62 / 92 -> 41 / 50 / 65), but the line stays below it: a single sequence
-// that fills the card runs as it does inside a larger batch, bit for bit. Below 256
-// positions a group would get one tile or two (T 256: 9 / 12 / 14 -> 10 / 11 /
-// 11). N = 256 has no LDS for a second group.
+// Forward / dQ / dK,dV, one group -> two (us, timed by events):
+//   N = 64   T 1024  128: 22 / 22 / 30 -> 18 / 19 / 23   248: 22 / 23 / 31 -> 18 / 21 / 25
+//            T 383   144: 14 / 14 / 19 -> 13 / 14 / 16   255: 14 / 15 / 19 -> 13 / 15 / 17
+//   N = 128  T 1024  128: 34 / 39 / 50 -> 28 / 34 / 38   248: 36 / 40 / 52 -> 31 / 36 / 41
+//            T 383   144: 20 / 24 / 29 -> 19 / 23 / 25   255: 21 / 25 / 30 -> 20 / 24 / 27
+// A second round of two-group workgroups costs more than two one-group ones on a
+// CU, which overlap by themselves: N = 128 T 383 288: 22 / 26 / 32 -> 25 / 33 / 37,
+// T 1024 288: 37 / 42 / 54 -> 33 / 44 / 51, 320: 39 / 48 / 62 -> 45 / 54 / 61,
+// 512: 41 / 51 / 65 -> 54 / 64 / 74; N = 64 T 1024 320: 24 / 29 / 37 -> 26 / 29 / 36.
+// Exactly one per CU still gains (T 1024 256: N = 64 22 / 23 / 30 -> 18 / 20 / 24,
+// N = 128 36 / 39 / 50 -> 30 / 35 / 39), but the line stays below it: a single
+// sequence that fills the card runs as it does inside a larger batch, bit for bit.
+// Calls on the two sides of the line differ in the rounding of their sums. At 256
+// positions a group gets one tile or two (N = 64 T 256 32: 12 / 13 / 15 -> 11 /
+// 12 / 14), below that none for the second. N = 256 has no LDS for a second group.
+// The line is the MI355X's 256 CUs as a constant, so that the rounding of a call
+// does not depend on the device it is asked of.
 constexpr int kSplitGrid = 256;
 inline bool attn_split(int grid, int len, int N) { return grid < kSplitGrid && len >= 256 && N <= 128; }
 hipError_t launch_attn_fwd(const AttnFwdParams& p, int N, hipStream_t s);

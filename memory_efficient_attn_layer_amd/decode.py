@@ -164,8 +164,10 @@ def _decode_launch(x3, weights, factor1, factor2, H, N, n_active, pos, cache, ep
 
 class DecodeGraph:
     """``decode_step`` captured once in a HIP graph for a fixed batch, cache and
-    set of weights, then replayed: one graph launch per step instead of five
-    kernel launches and the Python around them. ``step(x, pos)`` copies x
+    set of weights, then replayed: one graph launch per step instead of four
+    kernel launches and the Python around them (27 to 33 us of host time
+    either way; the input copies make the replayed step about 11 us longer
+    than the eager one). ``step(x, pos)`` copies x
     (B, C) and pos (B,) into the graph's static inputs, replays, and returns
     the static output (overwritten by the next step; clone it to keep it).
     Nothing in the captured step clears memory with a memset.
