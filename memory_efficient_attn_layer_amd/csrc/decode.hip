@@ -24,12 +24,12 @@
 // made it, so no workgroup waits for another's cache write.
 //
 // Measured (T = capacity, positions in its second half), attention with its
-// projection epilogue: B64 H8 N64 T4096 87 -> 74 us (403 MB, 5.4 TB/s), B16 H8
-// N128 T8192 95 -> 83, B1 H16 N128 T4096 13.1 -> 5.8 (a launch of its own for the
-// epilogue, splits of the capacity instead of the position and wave-private
-// stretches before). Requesting a wave's first block before the epilogue needs
-// 152 registers, three waves per SIMD: no faster (75.2 us), and spilled to 128
-// 124 us.
+// projection epilogue: B64 H8 N64 T4096 88 -> 75 us (403 MB, 5.4 TB/s), B16 H8
+// N128 T8192 89 -> 79, B1 H16 N128 T4096 15.8 -> 8.0, T65536 103 -> 88 (a launch
+// of its own for the epilogue, splits of the capacity instead of the position and
+// wave-private stretches before). Requesting a wave's first block before the
+// epilogue needs 152 registers, three waves per SIMD: no faster (75.2 us), and
+// spilled to 128 124 us.
 #include <type_traits>
 
 #include "common.cuh"
