@@ -177,9 +177,12 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
       d = row_sum<KL>(d);
       sc[i] = !TAIL || k0 + i * KPI + j < k_end ? d : -INFINITY;
     }
-    float mb = sc[0];
+    float mb = sc[0], lo = sc[0];
 #pragma unroll
-    for (int i = 1; i < NI; ++i) mb = fmaxf(mb, sc[i]);
+    for (int i = 1; i < NI; ++i) {
+      mb = fmaxf(mb, sc[i]);
+      lo = fminf(lo, sc[i]);
+    }
 #pragma unroll
     for (int off = KL; off < 64; off <<= 1) mb = fmaxf(mb, shfl_xor(mb, off));
     // The block's first key is valid, so mb is finite.
@@ -189,9 +192,18 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(DecodeParams p) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] *= alpha;
     m_run = m_new;
+    // The hardware exp2 takes results below 2^-126 for 0, exp2f does not.
+    float pr[NI];
+    if (__any(lo < m_new - 126.f)) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) pr[i] = exp2f(sc[i] - m_new);  // 0 for keys past the split
+    } else {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) pr[i] = fast_exp2(sc[i] - m_new);
+    }
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const float pv = exp2f(sc[i] - m_new);  // 0 for keys past the split
+      const float pv = pr[i];
       l_run += pv;
       float vf[8];
       unpack8(vr[i], vf);
